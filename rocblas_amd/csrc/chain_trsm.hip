@@ -2,9 +2,7 @@
 // and whose right-hand side is narrow: one workgroup per (64-row block I,
 // 16-vector panel p), chained through a completion counter per panel.
 //
-// Same canonical form and per-block arithmetic as the panel solve
-// (panel_trsm.hpp): forward substitution L y = c on the canonical lower
-// triangle, left-looking,
+// Canonical form as in panel_trsm.hpp; left-looking over 64-row blocks,
 //
 //   c_I = scale * b_I - sum_{J<I} L_IJ y_J    (FP64/FP32 MFMA)
 //   y_I = L_II^{-1} c_I                       (substitution, one DPP
@@ -37,7 +35,7 @@
 // stores) before the workgroup barrier that precedes the counter store; a
 // waiter polls with agent-scope loads and issues an agent-scope acquire fence
 // (cache invalidate) before reading y_J.
-#include "panel_trsm.hpp"
+#include "block_tile.hpp"
 
 namespace rbamd
 {
@@ -305,12 +303,14 @@ bool chain_fits(rocblas_handle h, int K, int nvec, int batch)
 {
     // Each block row streams its own tiles, so the tile traffic grows with
     // P * R^2 while the dependency chain grows with R: the chain pays off for
-    // small grids and for triangles long relative to the panel count (measured
+    // small grids and for triangles long relative to the panel count.  Up to
+    // kPanelMaxK rows the panel solve runs the whole chain inside a workgroup
+    // (512x256: 35 us, 59 chained).  (Measured
     // at 8x CUs: 4096x256 567 vs 937 us, 2048x512 336 vs 438 us recursive;
     // 1024x1024, P = 4R, 219 vs 183 us).
     const int64_t R = (K + PNB - 1) / PNB, P = (nvec + PNC - 1) / PNC;
     const int64_t cus = h->num_cus;
-    return h->chain_flags != nullptr && batch == 1 && K > 64 && R >= 2 && P <= kChainMaxPanels
+    return h->chain_flags != nullptr && batch == 1 && K > kPanelMaxK && P <= kChainMaxPanels
            && (R * P <= 2 * cus || (P <= R && R * P <= 8 * cus))
            && chain_lds_bytes(sizeof(T)) <= h->max_lds;
 }

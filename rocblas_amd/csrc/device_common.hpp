@@ -92,6 +92,19 @@ __device__ __forceinline__ void gstore(T* p, T v)
     *(__attribute__((address_space(1))) T*)(p) = v;
 }
 
+// lane N of each 16-lane row to the whole row
+template <int N>
+__device__ __forceinline__ double row_bcast(double x)
+{
+    return __builtin_amdgcn_mov_dpp(x, 0x150 + N, 0xf, 0xf, true);
+}
+
+template <int N>
+__device__ __forceinline__ float row_bcast(float x)
+{
+    return __builtin_amdgcn_mov_dpp(x, 0x150 + N, 0xf, 0xf, true);
+}
+
 // ---------------------------------------------------------------------------
 // Row broadcasts (row_newbcast: lane N of each 16-lane row to the whole row)
 // as inline assembly, shared by the small solve and the panel substitutions.

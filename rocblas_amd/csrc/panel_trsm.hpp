@@ -1,28 +1,44 @@
 // panel_trsm.hpp -- the panel solve shared by the single-launch k <= 512
 // path (panel_trsm.hip) and the persistent variable-size batch (vbatched.hip).
 //
-// panel_solve() solves 16 right-hand-side vectors [v0, v0 + 16) of one
-// instance with all 256 threads of the workgroup.  Canonical form as in
+// PanelSolver<T, NT, NVG> solves 16 * NVG right-hand-side vectors of one
+// instance with all four wavefronts of a workgroup.  Canonical form as in
 // small_trsm.hpp: forward substitution L y = c on the canonical lower triangle
 // (side L: vectors are columns of B, M = op(A); side R: vectors are rows of B,
-// M = op(A)^T; SF_REV reverses the index).  The triangle is walked in 64-row
-// blocks I, left-looking:
+// M = op(A)^T; SF_REV reverses the index).
 //
-//   c_I = scale * b_I - sum_{J<I} L_IJ y_J    (FP64/FP32 MFMA)
-//   y_I = L_II^{-1} c_I                       (substitution, DPP multiply-adds)
+// The triangle is cut into 16-row sub-blocks; wavefront w owns the sub-blocks
+// t = w (mod 4) of a super-block of up to 64 NT rows and keeps their updates
+// in registers, as MFMA accumulators, until each is solved (right-looking):
 //
-// Four wavefronts: in the update each owns 16 rows of the block (one 16x16
-// MFMA tile over the panel's 16 vectors); in the substitution each owns 4
-// vectors, a 16-lane row per vector, lane g holding rows g, g+16, g+32, g+48,
-// and every update of row i by the solved value of row j is one
-// v_fmac_dpp that broadcasts it from lane j%16 (row_newbcast).  Tiles of L
-// are staged through LDS with coalesced loads (either storage order of A),
-// the next tile's loads in flight during the current tile's MFMAs or
-// substitution.  The solved rows y_J are not kept: each block row reads them
-// back from B (where the substitution stored them), one tile ahead, so the
-// workgroup's LDS does not grow with K and two workgroups share a CU (which
-// hides each one's waits better than a deeper prefetch: the registers of a
-// second tile in flight would not fit two waves per SIMD).
+//   for e = 0, 1, ...:  s_t -= L_te y_e   for every own t > e   (MFMA)
+//   own t:              y_t = L_tt^{-1} (scale b_t + s_t)       (DPP substitution)
+//
+// Each entry of L feeds exactly one wavefront, so L goes from memory straight
+// to the MFMA operand registers: no LDS staging and no workgroup barrier in
+// the loop.  The solved sub-blocks are the only shared data: the owner writes
+// -y_t into a ring of LDS slots in operand order and raises a counter, and
+// the others poll that counter, so a wavefront waits only for what it needs --
+// the owner of the next sub-block applies y_{t-1} to that sub-block first,
+// solves and publishes it, and only then updates its other sub-blocks.
+//
+// MFMA operands: the product is formed as Y^T L^T, so the accumulator of a
+// sub-block is [vector][row]: lane l holds row l % 16, and register r a
+// vector of the 16-lane group l / 16.  That is the layout the substitution
+// wants: every 16-lane row of the wavefront holds the 16 rows of four vectors
+// (one per register), a step's solved values are broadcast from lane J by the
+// DPP multiply-add itself (row_newbcast), and the four registers are four
+// independent chains that hide each other's latency.  K slot q of product kk is
+// column 4 q + kk of L, so a lane's four values of y are contiguous in LDS.
+//
+// Bound: the chain of sub-blocks, about 1600 cycles per 16 rows (FP64, 16
+// vectors): 60 DPP multiply-adds (540), publishing through LDS (310),
+// noticing it (280), four dependent MFMAs (360) -- until, with many
+// sub-blocks left, the matrix cores are: 256 cycles per sub-block product.
+// Measured on MI355X against the solve this replaces (64-row blocks staged
+// through LDS, left-looking, workgroup barriers): FP64 256 instances
+// 200 x 64 79 -> 26 us, 512 x 512 on 6001 vectors 113 -> 57 us, one 512 x 256
+// solve 59 (chained over workgroups) -> 35 us.
 #pragma once
 
 #include "device_common.hpp"
@@ -31,378 +47,585 @@ namespace rbamd
 {
 namespace panel
 {
-constexpr int PNB   = 64;       // rows per block
-constexpr int PNC   = 16;       // vectors per panel
-constexpr int PLDA  = PNB + 1;  // LDS row stride of a staged tile
-constexpr int PLDY  = PNC + 1;  // LDS row stride of the solved panel
-constexpr int PNT   = 256;      // threads
-constexpr int PEPT  = PNB * PNB / PNT; // tile elements per thread
-constexpr int MCH   = 2;        // MFMA accumulator chains of a tile update
+constexpr int PNC   = 16;  // vectors per vector group, rows per sub-block
+constexpr int PNT   = 256; // threads
+constexpr int PRING = 8;   // LDS slots of solved sub-blocks
 
-// Fused substitution: Ln holds -L of the diagonal block with
-// its diagonal and upper part zero, rd[r] = 1 / L_ii of this lane's rows
-// i = g + 16 r.  Step J: the owner lane (g == J % 16) holds
-// x_J = c_J * rd_J in register q = J / 16, and each update is one
-// v_fmac_{f64,f32}_dpp broadcasting x_J from that lane:
-// c[r] += x_J * (-L[g + 16 r][J]).  Rows <= J are unchanged (their entries of
-// Ln are zero), so after the last step row i still holds c_i and
-// y_i = c_i * rd_i, which is x_i exactly as the step that owned row i computed it.
-// Registers r < q hold rows above J only, which are final: step J updates
-// (and loads the column entries of) registers q..3 alone.
-//
-// The inline-assembly updates are scheduling barriers, so the LDS reads of
-// column J are issued by hand FUSED_AHEAD steps early, into a ring of
-// FUSED_AHEAD + 1 register quadruples.
-constexpr int FUSED_AHEAD = 4;
-constexpr int FUSED_RING  = FUSED_AHEAD + 1;
-
-template <typename T, int J>
-__device__ __forceinline__ void fused_load(T (&l)[4], const T* Ln, int g)
+// Row pitch (elements) of a solved sub-block in LDS, [vector][row]: a lane
+// reads four consecutive rows of a vector as 16-byte words, conflict-free.
+template <typename T>
+constexpr int ypitch()
 {
-#pragma unroll
-    for(int r = J / 16; r < 4; ++r)
-        l[r] = Ln[(g + 16 * r) * PLDA + J];
+    return sizeof(T) == 8 ? 18 : 20;
 }
 
-template <typename T, int J>
-struct FusedSolve
+// LDS bytes of one workgroup: the ring, a diagonal block with its reciprocal
+// diagonal per wavefront, and the published-sub-block counter
+template <typename T, int NVG>
+constexpr size_t lds_bytes()
 {
-    static __device__ __forceinline__ void run(T (&c)[4], const T (&rd)[4], const T* Ln, int g,
-                                               int nrows, T (&lb)[FUSED_RING][4])
+    return sizeof(T) * PNC * (size_t(PRING) * NVG * ypitch<T>() + 4 * (ypitch<T>() + 1)) + 16;
+}
+
+// One substitution step for the four vectors a 16-lane row holds:
+// c_r += c_r[lane J] * l, with l = -L[g][J] / L[J][J] below the diagonal and 0
+// elsewhere.  A register is read through DPP four VALU instructions after the
+// previous step wrote it; the padding of step 0 covers whatever came before.
+template <int J>
+__device__ __forceinline__ void solve_step(double (&c)[4], double l)
+{
+    if constexpr(J == 0)
+        asm volatile("s_nop 4\n\t"
+                     "v_fmac_f64_dpp %0, %0, %4 row_newbcast:%5 row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t"
+                     "v_fmac_f64_dpp %1, %1, %4 row_newbcast:%5 row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t"
+                     "v_fmac_f64_dpp %2, %2, %4 row_newbcast:%5 row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t"
+                     "v_fmac_f64_dpp %3, %3, %4 row_newbcast:%5 row_mask:0xf bank_mask:0xf bound_ctrl:1"
+                     : "+v"(c[0]), "+v"(c[1]), "+v"(c[2]), "+v"(c[3])
+                     : "v"(l), "n"(J));
+    else
+        asm volatile("v_fmac_f64_dpp %0, %0, %4 row_newbcast:%5 row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t"
+                     "v_fmac_f64_dpp %1, %1, %4 row_newbcast:%5 row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t"
+                     "v_fmac_f64_dpp %2, %2, %4 row_newbcast:%5 row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t"
+                     "v_fmac_f64_dpp %3, %3, %4 row_newbcast:%5 row_mask:0xf bank_mask:0xf bound_ctrl:1"
+                     : "+v"(c[0]), "+v"(c[1]), "+v"(c[2]), "+v"(c[3])
+                     : "v"(l), "n"(J));
+}
+
+template <int J>
+__device__ __forceinline__ void solve_step(float (&c)[4], float l)
+{
+    if constexpr(J == 0)
+        asm volatile("s_nop 4\n\t"
+                     "v_fmac_f32_dpp %0, %0, %4 row_newbcast:%5 row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t"
+                     "v_fmac_f32_dpp %1, %1, %4 row_newbcast:%5 row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t"
+                     "v_fmac_f32_dpp %2, %2, %4 row_newbcast:%5 row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t"
+                     "v_fmac_f32_dpp %3, %3, %4 row_newbcast:%5 row_mask:0xf bank_mask:0xf bound_ctrl:1"
+                     : "+v"(c[0]), "+v"(c[1]), "+v"(c[2]), "+v"(c[3])
+                     : "v"(l), "n"(J));
+    else
+        asm volatile("v_fmac_f32_dpp %0, %0, %4 row_newbcast:%5 row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t"
+                     "v_fmac_f32_dpp %1, %1, %4 row_newbcast:%5 row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t"
+                     "v_fmac_f32_dpp %2, %2, %4 row_newbcast:%5 row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t"
+                     "v_fmac_f32_dpp %3, %3, %4 row_newbcast:%5 row_mask:0xf bank_mask:0xf bound_ctrl:1"
+                     : "+v"(c[0]), "+v"(c[1]), "+v"(c[2]), "+v"(c[3])
+                     : "v"(l), "n"(J));
+}
+
+template <typename T, int NVG, int J>
+struct SolveSteps
+{
+    static __device__ __forceinline__ void run(T (&c)[NVG][4], const T (&l)[PNC - 1])
     {
-        if constexpr(J < PNB)
+        if constexpr(J < PNC - 1) // row 15 has no rows below
         {
-            // rows past the block's last real row hold c = 0: their steps
-            // would add exact zeros (uniform branch)
-            if(J >= nrows)
-                return;
-            if constexpr(J + FUSED_AHEAD < PNB)
-                fused_load<T, J + FUSED_AHEAD>(lb[(J + FUSED_AHEAD) % FUSED_RING], Ln, g);
-            constexpr int q  = J / 16;
-            constexpr int jl = J % 16;
-            const T       x  = c[q] * rd[q];
-            T(&l)[4]         = lb[J % FUSED_RING];
-            // x was written just before the step's first update; the solve's
-            // very first update also covers a possible EXEC write
-            fmac_bcast<jl, J == 0 ? 5 : 2>(c[q], x, l[q]);
-            if constexpr(q < 1)
-                fmac_bcast<jl, 0>(c[1], x, l[1]);
-            if constexpr(q < 2)
-                fmac_bcast<jl, 0>(c[2], x, l[2]);
-            if constexpr(q < 3)
-                fmac_bcast<jl, 0>(c[3], x, l[3]);
-            FusedSolve<T, J + 1>::run(c, rd, Ln, g, nrows, lb);
+#pragma unroll
+            for(int v = 0; v < NVG; ++v)
+                solve_step<J>(c[v], l[J]);
+            SolveSteps<T, NVG, J + 1>::run(c, l);
         }
     }
 };
 
-// nrows: real rows of the block (steps nrows..63 are skipped)
-template <typename T>
-__device__ __forceinline__ void fused_solve(T (&c)[4], const T (&rd)[4], const T* Ln, int g,
-                                            int nrows)
+// Range in which a scaled entry -L[i][J] / L[J][J] stands for the division of
+// the step's value: finite, and not so small that bits of a non-zero entry
+// are lost.
+__device__ __forceinline__ bool scaled_ok(double l, double s)
 {
-    T lb[FUSED_RING][4];
-    fused_load<T, 0>(lb[0], Ln, g);
-    fused_load<T, 1>(lb[1], Ln, g);
-    fused_load<T, 2>(lb[2], Ln, g);
-    fused_load<T, 3>(lb[3], Ln, g);
-    static_assert(FUSED_AHEAD == 4, "prologue loads FUSED_AHEAD columns");
-    FusedSolve<T, 0>::run(c, rd, Ln, g, nrows, lb);
+    return (__builtin_fabs(s) <= 0x1p+1000) & ((__builtin_fabs(s) >= 0x1p-1000) | (l == 0.0));
+}
+__device__ __forceinline__ bool scaled_ok(float l, float s)
+{
+    return (__builtin_fabsf(s) <= 0x1p+120f) & ((__builtin_fabsf(s) >= 0x1p-120f) | (l == 0.0f));
 }
 
-// One 64 x 64 tile's update of a block's accumulators, sum_k L[row][k] y[k][v]
-// on MFMA: lrow = the tile in LDS at (16 w + lane % 16, lane / 16), ycol = the
-// solved block in LDS at (lane / 16, lane % 16) with row stride PLDY.  Each
-// half of the fragments is read before its first product; the products
-// alternate over MCH accumulator chains (fold_acc sums them).  The chained and panel solves both
-// accumulate through this function, so they round identically.
-template <typename T>
-__device__ __forceinline__ void mfma_tile(typename Mfma<T>::acc_t (&acc)[MCH], const T* lrow,
-                                          const T* ycol)
+// Bounds of the LDS waits.  Every wait ends by itself (all wavefronts of a
+// workgroup are resident, and the owner of the first unpublished sub-block
+// waits for published ones only); the poll limit turns a mistake into a
+// reported error instead of a hang: the wait raises the handle's error word
+// and goes on.  `bias` (0 in normal launches) makes every target unreachable.
+struct PanelWait
 {
-    constexpr int HALF = PNB / 8;
-#pragma unroll
-    for(int h = 0; h < 2; ++h)
-    {
-        T af[HALF], yf[HALF];
-#pragma unroll
-        for(int k = 0; k < HALF; ++k)
-        {
-            af[k] = lrow[4 * (h * HALF + k)];
-            yf[k] = ycol[4 * (h * HALF + k) * PLDY];
-        }
-#pragma unroll
-        for(int k = 0; k < HALF; ++k)
-            acc[k % MCH] = Mfma<T>::run(af[k], yf[k], acc[k % MCH]);
-    }
+    unsigned* err;
+    int       spin_limit;
+    int       bias;
+};
+
+inline PanelWait panel_wait(rocblas_handle h)
+{
+    return h->chain_debug_timeout ? PanelWait{h->async_error, 64, 1 << 30}
+                                  : PanelWait{h->async_error, 1 << 20, 0};
 }
 
+// vector of a group held in register r by 16-lane group q
 template <typename T>
-__device__ __forceinline__ T fold_acc(const typename Mfma<T>::acc_t (&acc)[MCH], int r)
+__device__ __forceinline__ int group_vec(int q, int r)
 {
-    static_assert(MCH == 2 || MCH == 4, "two or four chains");
-    if constexpr(MCH == 2)
-        return acc[0][r] + acc[1][r];
-    else
-        return (acc[0][r] + acc[1][r]) + (acc[2][r] + acc[3][r]);
+    return Mfma<T>::row(q << 4, r);
 }
 
-// LDS bytes of one workgroup (the same for every triangle size)
+// B := 0 for nv vectors from v0 (alpha == 0; A is not referenced)
 template <typename T>
-__host__ __device__ constexpr size_t lds_bytes(int /*K*/)
+__device__ void panel_zero(T* Bp, int K, int nvec, int ldb, int flags, int v0, int nv)
 {
-    return sizeof(T) * (size_t(PNB) * PLDA + size_t(PNB) * PNC + PNB + size_t(PNB) * PLDY);
-}
-
-// B := 0 for the panel's vectors (alpha == 0; A is not referenced)
-template <typename T>
-__device__ void panel_zero(T* Bp, int K, int nvec, int ldb, int flags, int v0)
-{
-    const bool rev  = flags & SF_REV;
     const bool cols = flags & SF_COLS;
-    for(int e = threadIdx.x; e < K * PNC; e += PNT)
+    for(int e = threadIdx.x; e < K * nv; e += PNT)
     {
-        const int i = e % K, v = v0 + e / K;
-        const int r = rev ? K - 1 - i : i;
+        const int i = cols ? e % K : e / nv, v = v0 + (cols ? e / K : e % nv);
         if(v < nvec)
-            gstore(Bp + (cols ? int64_t(r) + int64_t(v) * ldb : int64_t(v) + int64_t(r) * ldb),
+            gstore(Bp + (cols ? int64_t(i) + int64_t(v) * ldb : int64_t(v) + int64_t(i) * ldb),
                    T(0));
     }
 }
 
-template <typename T>
-__device__ void panel_solve(const T* __restrict__ Ap, T* Bp, int K, int nvec, int lda, int ldb,
-                            int flags, T scale, int v0, unsigned char* smem)
+// MULTI: K may exceed 64 NT rows (several super-blocks).
+template <typename T, int NT, int NVG, bool MULTI>
+struct PanelSolver
 {
-    T* Ls    = reinterpret_cast<T*>(smem); // PNB x PLDA staged tile
-    T* Cs    = Ls + PNB * PLDA;            // PNB x PNC accumulated update
-    T* rdiag = Cs + PNB * PNC;             // PNB reciprocal diagonal
-    T* Yt    = rdiag + PNB;                // PNB x PLDY solved block y_J of the tile
+    using acc_t             = typename Mfma<T>::acc_t;
+    static constexpr int YP = ypitch<T>();
+    static constexpr int YV = PNC * YP;  // elements of one vector group in a slot
+    static constexpr int YS = NVG * YV;  // elements of one slot
 
-    const int  tid  = threadIdx.x;
-    const int  lane = tid & (WAVE - 1);
-    const int  w    = tid / WAVE;
-    const bool tA   = flags & SF_TA;
-    const bool rev  = flags & SF_REV;
-    const bool unit = flags & SF_UNIT;
-    const bool cols = flags & SF_COLS;
-    const int  nblk = (K + PNB - 1) / PNB;
+    // instance: canonical L(i, j) at Ab[i rs + j cs], right-hand side (row i,
+    // vector v) at Bb[i br + v bv]
+    const T* Ab;
+    T*       Bb;
+    int      rs, cs, br, bv;
+    int      K, nsub, nvec, v0;
+    bool     unit;
+    T        scale;
+    // wavefront and lane
+    int     w, g, q;
+    int64_t lq; // 4 q columns
+    // LDS
+    T*        Y;
+    T*        D; // this wavefront's diagonal block and reciprocal diagonal
+    int*      done;
+    int       seen;
+    PanelWait pw;
 
-    // substitution layout: vector vl = 4w + lane/16, rows g + 16r of a block
-    const int  g   = lane & 15;
-    const int  vl  = 4 * w + (lane >> 4);
-    const int  vec = v0 + vl;
-    const bool vok = vec < nvec;
+    // state: -sum of L y so far, L operands in flight; of the next sub-block to
+    // solve the right-hand sides and the diagonal block
+    acc_t C[NT][NVG];
+    T     Lf[NT][4];
+    T     bq[NVG][4];
+    T     Dr[4];       // the diagonal block as loaded
+    T     dg;          // and this lane's diagonal entry, then its reciprocal
+    int   sb; // first sub-block of the super-block
+    int   e;  // next solved sub-block to apply
 
-    auto boff = [&](int i, int v) -> int64_t {
-        const int r = rev ? K - 1 - i : i;
-        return cols ? int64_t(r) + int64_t(v) * ldb : int64_t(v) + int64_t(r) * ldb;
-    };
-
-    // Tile (I, J) of canonical L, element s of this thread: canonical
-    // (i, j) = (lane, wu + 4s) (A read as is) or (wu + 4s, lane) (A^T), so
-    // that consecutive lanes read consecutive addresses.  The lane's index
-    // fixes the address within a column of A's storage and the wavefront's
-    // (wu + 4s) picks the column, which is wave-uniform: each element is one
-    // load at a scalar column address plus the lane's fixed offset.
-    const int wu      = __builtin_amdgcn_readfirstlane(w);
-    auto      tile_ij = [&](int s, int& i, int& j) {
-        i = tA ? wu + 4 * s : lane;
-        j = tA ? lane : wu + 4 * s;
-    };
-    auto fold = [&](int x) { return rev ? K - 1 - x : x; };
-    // Raw values of a tile in flight.  Indices past K - 1 read row (column)
-    // K - 1 instead, so every load is in bounds and unpredicated; only the
-    // last block row has such rows, and their results are never used.
-    auto load_tile = [&](T(&reg)[PEPT], int I, int J) {
-        const int p  = fold(min((tA ? J : I) * PNB + lane, K - 1)); // lane's row in A
-        const int qb = (tA ? I : J) * PNB + wu;
-#pragma unroll
-        for(int s = 0; s < PEPT; ++s)
-        {
-            const int q = fold(min(qb + 4 * s, K - 1)); // the column, wave-uniform
-            reg[s]      = gload(Ap + int64_t(q) * lda + p);
-        }
-    };
-    // An off-diagonal tile (J < I) is dense and its columns are all below K;
-    // rows past K (last block row) carry row K - 1's values into MFMA result
-    // rows that are discarded, so it is stored without a mask.
-    // (two loops, so each element's LDS address is an immediate offset from
-    // one base register)
-    T* const lds0       = Ls + (tA ? wu * PLDA + lane : lane * PLDA + wu); // element 0
-    auto     store_tile = [&](const T(&reg)[PEPT]) {
-        if(tA)
-        {
-#pragma unroll
-            for(int s = 0; s < PEPT; ++s)
-                lds0[s * 4 * PLDA] = reg[s];
-        }
-        else
-        {
-#pragma unroll
-            for(int s = 0; s < PEPT; ++s)
-                lds0[s * 4] = reg[s];
-        }
-    };
-    // the diagonal block: -L strictly below the diagonal (the fused
-    // substitution's operand), the diagonal into rdiag
-    auto store_diag = [&](const T(&reg)[PEPT], int I) {
-#pragma unroll
-        for(int s = 0; s < PEPT; ++s)
-        {
-            int i, j;
-            tile_ij(s, i, j);
-            const int gi = I * PNB + i;
-            Ls[i * PLDA + j] = (gi < K && j < i) ? -reg[s] : T(0);
-            if(i == j)
-                rdiag[i] = (gi < K && !unit) ? reg[s] : T(1);
-        }
-    };
-    // right-hand sides of block row I; rows past K and vectors past nvec
-    // read an element in bounds (row K - 1, vector nvec - 1), discarded
-    // later, so the loads need no branch
-    const int vclamp = min(vec, nvec - 1);
-    auto      load_rhs = [&](T(&bv)[4], int I) {
-#pragma unroll
-        for(int r = 0; r < 4; ++r)
-            bv[r] = gload(Bp + boff(min(I * PNB + g + 16 * r, K - 1), vclamp));
-    };
-
-    // y_J of block row J for the panel's vectors, read back from B: 64 rows x
-    // 16 vectors, four per thread, consecutive lanes along B's contiguous
-    // dimension.  Rows past K and vectors past nvec read row K - 1 / vector
-    // nvec - 1 (in bounds; such values never reach a stored result).
-    auto y_rv = [&](int s, int& r, int& v) {
-        const int e = tid + PNT * s;
-        r           = cols ? e % PNB : e / PNC;
-        v           = cols ? e / PNB : e % PNC;
-    };
-    auto load_y = [&](T(&yv)[4], int J) {
-#pragma unroll
-        for(int s = 0; s < 4; ++s)
-        {
-            int r, v;
-            y_rv(s, r, v);
-            yv[s] = gload(Bp + boff(min(J * PNB + r, K - 1), min(v0 + v, nvec - 1)));
-        }
-    };
-    auto store_y = [&](const T(&yv)[4]) {
-#pragma unroll
-        for(int s = 0; s < 4; ++s)
-        {
-            int r, v;
-            y_rv(s, r, v);
-            Yt[r * PLDY + v] = yv[s];
-        }
-    };
-    static_assert(PNB * PNC == 4 * PNT, "four y values per thread");
-
-    // The tiles are consumed in the order (0,0), (1,0), (1,1), (2,0), ...,
-    // (I, I) being the diagonal block that ends block row I.  The register
-    // buffer ra is refilled with the next tile as soon as its tile is in
-    // LDS, so each tile's load latency overlaps the step before it is needed.
-    // Every step issues exactly one tile's loads (past the last tile, the
-    // last tile again, never consumed), so each path through a step leaves
-    // the same number of loads in flight and the compiler's wait counts
-    // retire only the tile being consumed.
-    int  iI = 0, iJ = 0; // next tile to load
-    auto issue = [&](T(&reg)[PEPT]) {
-        const bool past = iI >= nblk;
-        load_tile(reg, past ? nblk - 1 : iI, past ? nblk - 1 : iJ);
-        if(!past && ++iJ > iI)
-        {
-            ++iI;
-            iJ = 0;
-        }
-    };
-    T ra[PEPT];
-    issue(ra);
-    T yv[4]; // y of the next off-diagonal tile (loaded one step ahead)
-
-    int cI = 0, cJ = 0; // tile being consumed
-    typename Mfma<T>::acc_t acc[MCH];
-#pragma unroll
-    for(int a = 0; a < MCH; ++a)
-        acc[a] = typename Mfma<T>::acc_t{0, 0, 0, 0};
-    const T* lrow = Ls + (16 * w + (lane & 15)) * PLDA + (lane >> 4);
-    const T* ycol = Yt + (lane >> 4) * PLDY + (lane & 15);
-
-    // consume the tile held in `reg`; true once the last block row is solved
-    auto step = [&](T(&reg)[PEPT]) -> bool {
-        if(cJ < cI)
-        {
-            // ---- c_I accumulation: L_IJ y_J on MFMA ----
-            __syncthreads(); // previous readers of Ls and Yt are done
-            store_tile(reg);
-            store_y(yv);
-            __syncthreads();
-            issue(reg);
-            // y of the next tile: y_{J+1}, or (the diagonal tile is next) a
-            // load nobody reads, so every step issues the same loads
-            load_y(yv, cJ + 1 < cI ? cJ + 1 : 0);
-            mfma_tile<T>(acc, lrow, ycol);
-            ++cJ;
-            return false;
-        }
-        // diagonal block (I, I): -L below the diagonal, reciprocal diagonal.
-        // The block row's right-hand sides are loaded first: only the next
-        // tile's loads follow them, so waiting for them drains no prefetch
-        T bv[4];
-        load_rhs(bv, cI);
-        __syncthreads();
-        store_diag(reg, cI);
-#pragma unroll
-        for(int r = 0; r < 4; ++r)
-            Cs[(16 * w + Mfma<T>::row(lane, r)) * PNC + (lane & 15)] = fold_acc<T>(acc, r);
-        __syncthreads();
-        if(tid < PNB)
-            rdiag[tid] = T(1) / rdiag[tid];
-        __syncthreads();
-        issue(reg);
-
-        // ---- y_I = L_II^{-1} c_I ----
-        T c[4], rd[4];
-#pragma unroll
-        for(int r = 0; r < 4; ++r)
-        {
-            const int  gi = cI * PNB + g + 16 * r;
-            const bool ok = vok && gi < K;
-            c[r]          = ok ? scale * bv[r] - Cs[(g + 16 * r) * PNC + vl] : T(0);
-            rd[r]         = rdiag[g + 16 * r];
-        }
-        // every operand of the DPP updates is final here (an empty asm that
-        // redefines it), so no VALU instruction producing one of them is
-        // sunk in front of its first DPP reader
-#pragma unroll
-        for(int r = 0; r < 4; ++r)
-        {
-            asm volatile("" : "+v"(c[r]));
-            asm volatile("" : "+v"(rd[r]));
-        }
-        fused_solve<T>(c, rd, Ls, g, min(PNB, K - cI * PNB));
-#pragma unroll
-        for(int r = 0; r < 4; ++r)
-        {
-            const int gi = cI * PNB + g + 16 * r;
-            if(gi < K && vok)
-                gstore(Bp + boff(gi, vec), c[r] * rd[r]);
-        }
-        ++cI;
-        cJ = 0;
-        if(cI >= nblk)
-            return true;
-        // every wavefront's rows of y_I are in B before any is read back
-        __syncthreads();
-        load_y(yv, 0); // the next tile is (I + 1, 0)
-#pragma unroll
-        for(int a = 0; a < MCH; ++a)
-            acc[a] = typename Mfma<T>::acc_t{0, 0, 0, 0};
-        return false;
-    };
-    while(!step(ra))
+    __device__ __forceinline__ int tile(int mine, int act) const
     {
+        return sb + w + 4 * (mine - act);
     }
-    __syncthreads(); // LDS reuse by the caller's next panel
-}
+
+    // One address register pair, stepped from load to load: a set of
+    // addresses computed ahead would need more registers than the operands.
+    static __device__ __forceinline__ void pin(const T*& p)
+    {
+        asm volatile("" : "+v"(p));
+    }
+
+    // operand registers of L(t, ev): row 16 t + g, columns 16 ev + 4 q + kk.
+    // Rows past K - 1 (last sub-block) read row K - 1; they feed only rows
+    // that are never stored.  ev < t, so every column is below K.
+    __device__ __forceinline__ void load_l(T (&f)[4], int t, int ev)
+    {
+        const int row = min(PNC * t + g, K - 1);
+        const T*  p   = Ab + int64_t(PNC * ev) * cs + (int64_t(row) * rs + lq);
+#pragma unroll
+        for(int kk = 0; kk < 4; ++kk)
+        {
+            f[kk] = gload(p);
+            p += cs;
+            pin(p);
+        }
+    }
+
+    // raw diagonal block of sub-block t: row 16 t + g, columns 16 t + 4 q + kk,
+    // and the row's diagonal entry (indices past K - 1 read K - 1 instead)
+    __device__ __forceinline__ void load_diag(int t)
+    {
+        const int row = min(PNC * t + g, K - 1);
+        const T*  p   = Ab + int64_t(row) * rs;
+        dg            = gload(p + int64_t(row) * cs);
+#pragma unroll
+        for(int kk = 0; kk < 4; ++kk)
+            Dr[kk] = gload(p + int64_t(min(PNC * t + 4 * q + kk, K - 1)) * cs);
+    }
+
+    // Diagonal block of sub-block t: its reciprocal diagonal, and its columns
+    // below the diagonal scaled by it (0 elsewhere, and in rows past K - 1,
+    // whose entries may lie outside the triangle), row g in every lane of
+    // column g.  Each lane scales the four entries it loaded, and a wavefront's
+    // own 16 x 16 corner of LDS spreads the rows (a wavefront's LDS accesses
+    // execute in order).  False if an entry leaves the range (a nearly
+    // singular or badly scaled block): solve() then takes the unscaled form.
+    // Pinned, so that all of it is done before the wait for the last update.
+    __device__ __forceinline__ bool prep_diag(T (&Ld)[PNC - 1], int t)
+    {
+        constexpr int PER = 16 / int(sizeof(T));
+        typedef T     word __attribute__((ext_vector_type(PER)));
+        const int     below = PNC * t + g < K ? g : 0;
+        T* const      rd    = D + PNC * YP;
+        dg                  = unit ? T(1) : T(1) / dg;
+        rd[g]               = dg;
+        asm volatile("" ::: "memory");
+        bool ok = true;
+        T    s[4];
+#pragma unroll
+        for(int kk = 0; kk < 4; ++kk)
+        {
+            const bool low = 4 * q + kk < below;
+            const T    x   = low ? -Dr[kk] : T(0);
+            s[kk]          = x * rd[4 * q + kk];
+            ok             = ok & (!low | scaled_ok(x, s[kk]));
+            s[kk]          = low ? s[kk] : T(0);
+        }
+        T* const dw = D + g * YP;
+#pragma unroll
+        for(int k0 = 0; k0 < 4; k0 += PER)
+        {
+            word x;
+#pragma unroll
+            for(int i = 0; i < PER; ++i)
+                x[i] = s[k0 + i];
+            *reinterpret_cast<word*>(dw + 4 * q + k0) = x;
+        }
+        const bool all = __builtin_amdgcn_ballot_w64(!ok) == 0;
+        asm volatile("" ::: "memory");
+#pragma unroll
+        for(int j = 0; j < PNC; j += PER)
+        {
+            const word x = *reinterpret_cast<const word*>(dw + j);
+#pragma unroll
+            for(int i = 0; i < PER; ++i)
+                if(j + i < PNC - 1)
+                    Ld[j + i] = x[i];
+        }
+#pragma unroll
+        for(int j = 0; j < PNC - 1; ++j)
+            asm volatile("" : "+v"(Ld[j]));
+        return all;
+    }
+
+    // right-hand sides of sub-block t
+    __device__ __forceinline__ void load_rhs(int t)
+    {
+        const T* p = Bb + int64_t(min(PNC * t + g, K - 1)) * br;
+#pragma unroll
+        for(int v = 0; v < NVG; ++v)
+#pragma unroll
+            for(int r = 0; r < 4; ++r)
+                bq[v][r]
+                    = gload(p + int64_t(min(v0 + PNC * v + group_vec<T>(q, r), nvec - 1)) * bv);
+    }
+
+    // y of sub-block ev of an earlier super-block, read back from B (negated)
+    __device__ __forceinline__ void load_y(T (&y)[NVG][4], int ev)
+    {
+#pragma unroll
+        for(int v = 0; v < NVG; ++v)
+        {
+            const T* p = Bb + int64_t(min(v0 + PNC * v + g, nvec - 1)) * bv
+                         + int64_t(PNC * ev + 4 * q) * br;
+#pragma unroll
+            for(int kk = 0; kk < 4; ++kk)
+                y[v][kk] = gload(p + int64_t(kk) * br);
+        }
+    }
+
+    // y of sub-block ev, once it is published.  Each poll reads the counter
+    // and then the slot: a wavefront's LDS reads execute in order, so when the
+    // counter says the slot is written, the values read after it are the
+    // published ones (otherwise they are read again).
+    __device__ __forceinline__ void wait_y(T (&yf)[NVG][4], int ev)
+    {
+        // 16-byte words (every term of the address is a multiple of one)
+        constexpr int PER = 16 / int(sizeof(T));
+        typedef T     word __attribute__((ext_vector_type(PER)));
+        const T*      p    = Y + (ev % PRING) * YS + g * YP + 4 * q;
+        const int     need = ev + 1 + pw.bias;
+        for(int it = 0;; ++it)
+        {
+            int n = seen;
+            if(n < need)
+                n = __hip_atomic_load(done, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+            asm volatile("" ::: "memory"); // the slot is read after the counter
+#pragma unroll
+            for(int v = 0; v < NVG; ++v)
+#pragma unroll
+                for(int k0 = 0; k0 < 4; k0 += PER)
+                {
+                    const word x = *reinterpret_cast<const word*>(p + v * YV + k0);
+#pragma unroll
+                    for(int i = 0; i < PER; ++i)
+                        yf[v][k0 + i] = x[i];
+                }
+            seen = __builtin_amdgcn_readfirstlane(n);
+            if(seen >= need)
+                break;
+            if(it >= pw.spin_limit)
+            {
+                if(pw.err)
+                    __hip_atomic_store(pw.err, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+                seen = 0x7fffffff;
+                break;
+            }
+            asm volatile("" ::: "memory");
+        }
+    }
+
+    // c_t += (-y)^T L^T
+    template <int I>
+    __device__ __forceinline__ void apply(const T (&yf)[NVG][4])
+    {
+#pragma unroll
+        for(int kk = 0; kk < 4; ++kk)
+#pragma unroll
+            for(int v = 0; v < NVG; ++v)
+                C[I][v] = Mfma<T>::run(yf[v][kk], Lf[I][kk], C[I][v]);
+    }
+
+    // apply the current y to own tiles I..NT-1 and load their next operands
+    // (tile I is sub-block t, the others follow 4 apart)
+    template <int I>
+    __device__ __forceinline__ void apply_from(const T (&yf)[NVG][4], int t)
+    {
+        if constexpr(I < NT)
+        {
+            apply<I>(yf);
+            load_l(Lf[I], t, e + 1);
+            apply_from<I + 1>(yf, t + 4);
+        }
+    }
+
+    // The unscaled substitution, for blocks prep_diag() refuses: x_J = c_J / L_JJ
+    // first, then c_i -= L_iJ x_J, column by column from memory.
+    __device__ __forceinline__ void solve_unscaled(T (&c)[NVG][4], int t)
+    {
+        const int below = PNC * t + g < K ? g : 0;
+        const T*  p     = Ab + int64_t(min(PNC * t + g, K - 1)) * rs + int64_t(PNC * t) * cs;
+        for(int j = 0; j < PNC - 1 && PNC * t + j < K; ++j)
+        {
+            const T x = gload(p + int64_t(j) * cs);
+            const T l = j < below ? -x : T(0);
+#pragma unroll
+            for(int v = 0; v < NVG; ++v)
+#pragma unroll
+                for(int r = 0; r < 4; ++r)
+                    c[v][r] = fma(__shfl(c[v][r] * dg, 16 * q + j, WAVE), l, c[v][r]);
+        }
+    }
+
+    // own sub-block t (tile I) is final: solve, publish, store
+    template <int I>
+    __device__ __forceinline__ void solve(const T (&Ld)[PNC - 1], int t, bool scaled)
+    {
+        // the accumulated sums join the right-hand sides only here, so their
+        // roundings are of the sums' own size (and the MFMA results are first
+        // read by instructions the compiler pads for: it does not look into
+        // inline assembly)
+        T c[NVG][4];
+#pragma unroll
+        for(int v = 0; v < NVG; ++v)
+#pragma unroll
+            for(int r = 0; r < 4; ++r)
+                c[v][r] = fma(scale, bq[v][r], C[I][v][r]);
+        if(scaled)
+            SolveSteps<T, NVG, 0>::run(c, Ld);
+        else
+            solve_unscaled(c, t);
+        T* p = Y + (t % PRING) * YS + g;
+#pragma unroll
+        for(int v = 0; v < NVG; ++v)
+#pragma unroll
+            for(int r = 0; r < 4; ++r)
+            {
+                c[v][r] *= dg;
+                p[v * YV + group_vec<T>(q, r) * YP] = -c[v][r];
+            }
+        // the slot is written before the counter says so
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        __hip_atomic_store(done, t + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        // (opaque, so the addresses are not kept in registers all along)
+        int qs = q;
+        asm volatile("" : "+v"(qs));
+        const int row = PNC * t + g;
+        T*        b   = Bb + int64_t(row) * br;
+#pragma unroll
+        for(int v = 0; v < NVG; ++v)
+#pragma unroll
+            for(int r = 0; r < 4; ++r)
+            {
+                const int vec = v0 + PNC * v + group_vec<T>(qs, r);
+                if(row < K && vec < nvec)
+                    gstore(b + int64_t(vec) * bv, c[v][r]);
+            }
+    }
+
+    // Own tiles are C[NT - mine]..C[NT - 1].  Tile I is the first one not yet
+    // solved (if this wavefront has so many): bring it up to date, solve it,
+    // go on with the others.
+    template <int I>
+    __device__ __forceinline__ void segments(int mine)
+    {
+        if constexpr(I < NT)
+        {
+            if(mine >= NT - I)
+            {
+                const int t = sb + w + 4 * (mine - (NT - I));
+                T         yf[NVG][4];
+                T         Ld[PNC - 1];
+                for(; e < t - 1; ++e)
+                {
+                    wait_y(yf, e);
+                    apply_from<I>(yf, t);
+                }
+                const bool scaled = prep_diag(Ld, t);
+                if(t > sb)
+                {
+                    wait_y(yf, e); // e == t - 1
+                    apply<I>(yf);
+                }
+                solve<I>(Ld, t, scaled);
+                if(I + 1 < NT)
+                {
+                    load_diag(t + 4);
+                    load_rhs(t + 4);
+                    if(t > sb)
+                    {
+                        apply_from<I + 1>(yf, t + 4);
+                        ++e;
+                    }
+                }
+            }
+            segments<I + 1>(mine);
+        }
+    }
+
+    __device__ __forceinline__ void clear(int i)
+    {
+#pragma unroll
+        for(int v = 0; v < NVG; ++v)
+            C[i][v] = acc_t{0, 0, 0, 0};
+#pragma unroll
+        for(int kk = 0; kk < 4; ++kk)
+            Lf[i][kk] = T(0);
+    }
+
+    // a super-block in which this wavefront owns `mine` sub-blocks
+    __device__ __forceinline__ void super_block(int mine)
+    {
+        const int t0 = sb + w;
+        dg = T(0);
+#pragma unroll
+        for(int kk = 0; kk < 4; ++kk)
+            Dr[kk] = T(0);
+#pragma unroll
+        for(int v = 0; v < NVG; ++v)
+#pragma unroll
+            for(int r = 0; r < 4; ++r)
+                bq[v][r] = T(0);
+        if(mine > 0)
+        {
+            load_diag(t0);
+            load_rhs(t0);
+        }
+#pragma unroll
+        for(int i = 0; i < NT; ++i)
+        {
+            clear(i); // (nothing is carried over from an earlier solve)
+            if(mine >= NT - i)
+            {
+                const int t = t0 + 4 * (mine - (NT - i));
+                if(t > 0)
+                    load_l(Lf[i], t, 0);
+            }
+        }
+        e = 0;
+        if(MULTI && sb > 0)
+        {
+            // the earlier super-blocks' solution, without a chain
+            T yf[NVG][4], yn[NVG][4];
+            load_y(yn, 0);
+            for(; e < sb; ++e)
+            {
+#pragma unroll
+                for(int v = 0; v < NVG; ++v)
+#pragma unroll
+                    for(int kk = 0; kk < 4; ++kk)
+                        yf[v][kk] = -yn[v][kk];
+                load_y(yn, min(e + 1, sb - 1));
+                early<0>(yf, mine);
+            }
+        }
+        segments<0>(mine);
+    }
+
+    // one sub-block of an earlier super-block, applied to every own tile
+    template <int I>
+    __device__ __forceinline__ void early(const T (&yf)[NVG][4], int mine)
+    {
+        if constexpr(I < NT)
+        {
+            if(mine >= NT - I)
+            {
+                const int t = sb + w + 4 * (mine - (NT - I));
+                apply<I>(yf);
+                if(e + 1 < t)
+                    load_l(Lf[I], t, e + 1);
+            }
+            early<I + 1>(yf, mine);
+        }
+    }
+
+    __device__ __forceinline__ void run(const T* Ap, T* Bp, int K_, int nvec_, int lda, int ldb,
+                                        int flags, T scale_, int v0_, unsigned char* smem,
+                                        PanelWait pw_)
+    {
+        const bool tA   = flags & SF_TA;
+        const bool rev  = flags & SF_REV;
+        const bool cols = flags & SF_COLS;
+        const int  lane = threadIdx.x & (WAVE - 1);
+        K               = K_;
+        nsub            = (K + PNC - 1) / PNC;
+        nvec            = nvec_;
+        v0              = v0_;
+        unit            = flags & SF_UNIT;
+        scale           = scale_;
+        w               = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
+        g               = lane & 15;
+        q               = lane >> 4;
+        const int s     = rev ? -1 : 1;
+        rs              = s * (tA ? lda : 1);
+        cs              = s * (tA ? 1 : lda);
+        br              = s * (cols ? 1 : ldb);
+        bv              = cols ? ldb : 1;
+        lq              = int64_t(4 * q) * cs;
+        Ab              = Ap + (rev ? int64_t(K - 1) * (int64_t(lda) + 1) : 0);
+        Bb              = Bp + (rev ? int64_t(K - 1) * (cols ? 1 : ldb) : 0);
+        Y               = reinterpret_cast<T*>(smem);
+        D               = Y + PRING * YS + w * PNC * (YP + 1);
+        done            = reinterpret_cast<int*>(Y + PRING * YS + 4 * PNC * (YP + 1));
+        pw              = pw_;
+        seen            = 0;
+        if(threadIdx.x == 0)
+            *done = 0;
+        __syncthreads();
+        sb = 0;
+        if constexpr(!MULTI)
+            super_block((nsub - w + 3) / 4);
+        else
+            for(; sb < nsub; sb += 4 * NT)
+            {
+                // the earlier super-blocks' stores to B are visible, the ring is free
+                if(sb > 0)
+                    __syncthreads();
+                super_block((min(4 * NT, nsub - sb) - w + 3) / 4);
+            }
+        __syncthreads(); // LDS reuse by the caller's next panel
+    }
+};
 } // namespace panel
 } // namespace rbamd

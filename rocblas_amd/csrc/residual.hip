@@ -21,7 +21,7 @@
 // are FP64 atomic adds, so their order -- and eta's last bits -- can vary from
 // run to run; eta is a measurement, not a result.
 #include "device_common.hpp"
-#include "panel_trsm.hpp"
+#include "block_tile.hpp"
 #include "residual.hpp"
 
 namespace rbamd

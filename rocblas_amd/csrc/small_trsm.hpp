@@ -333,18 +333,6 @@ __global__ void __launch_bounds__(WAVE) small_trsm_lds_kernel(const SmallArgs<T>
 constexpr int DPP_VP = 16; // vectors per slot
 constexpr int DPP_G  = 4;  // slots per wavefront
 
-template <int N>
-__device__ __forceinline__ double row_bcast(double x)
-{
-    return __builtin_amdgcn_mov_dpp(x, 0x150 + N, 0xf, 0xf, true);
-}
-
-template <int N>
-__device__ __forceinline__ float row_bcast(float x)
-{
-    return __builtin_amdgcn_mov_dpp(x, 0x150 + N, 0xf, 0xf, true);
-}
-
 template <typename T, int KMAX>
 using DppTri = T[(KMAX * (KMAX + 1) / 2 + 15) / 16];
 

@@ -331,12 +331,7 @@ struct Solver
         return launch_gemm(h, g);
     }
 
-    // SMALL_K < k <= kPanelMaxK: one launch solves the whole range -- the
-    // chained kernel for one instance whose leaf has at most two vector
-    // panels per 64-row block (a 512-row leaf of 256 vectors: 8 x 16
-    // workgroups instead of 16; with more panels the chain's waits cost more
-    // than the extra workgroups gain: 2048^2 769 vs 499 us), else one
-    // workgroup per panel; both give the same bits
+    // SMALL_K < k <= kPanelMaxK: one launch solves the whole range
     rocblas_status panel_leaf(int a, int b)
     {
         const int    K  = b - a;
@@ -352,9 +347,6 @@ struct Solver
                   | (p.diag == rocblas_diagonal_unit ? SF_UNIT : 0) | (sideL ? SF_COLS : 0);
         s.alpha_host = T(1);
         s.alpha_dev  = p.alpha_dev; // only the alpha == 0 guard
-        const int blocks = (K + 63) / 64, panels = (s.nvec + 15) / 16;
-        if(panels <= 2 * blocks && chain_fits<T>(h, K, s.nvec, p.batch))
-            return launch_chain<T>(h, s);
         return launch_panel<T>(h, s, p.batch);
     }
 
@@ -421,8 +413,9 @@ rocblas_status trsm_launch(rocblas_handle h, const TrsmProblem<T>& p)
 
     if(chain_fits<T>(h, K, sideL ? p.n : p.m, p.batch) || panel_fits<T>(h, K))
     {
-        // one launch that scales by alpha itself: chained blocks for one
-        // instance with few vector panels, else one workgroup per panel
+        // one launch that scales by alpha itself: one workgroup per 16 or 32
+        // vectors up to kPanelMaxK rows, chained blocks for one longer
+        // instance with few vector panels
         SmallArgs<T> s{};
         s.A          = p.A;
         s.B          = p.B;

@@ -162,9 +162,9 @@ __global__ void __launch_bounds__(1024) vb_plan_kernel(const VbArgs<T> a)
 // Panel kernel: persistent workgroups over the panel work items.
 template <typename T>
 __global__ void __launch_bounds__(panel::PNT) __attribute__((amdgpu_waves_per_eu(2)))
-    vb_panel_kernel(const VbArgs<T> a)
+    vb_panel_kernel(const VbArgs<T> a, panel::PanelWait pw)
 {
-    extern __shared__ __align__(16) unsigned char vb_smem[];
+    __shared__ __align__(16) unsigned char vb_smem[panel::lds_bytes<T, 1>()];
     __shared__ int item_s;
     const int      total = a.counter[1];
     if(int(blockIdx.x) >= total)
@@ -200,10 +200,12 @@ __global__ void __launch_bounds__(panel::PNT) __attribute__((amdgpu_waves_per_eu
         for(int p = g; p < panels; p += G)
         {
             if(alpha == T(0))
-                panel::panel_zero<T>(Bp, k, nv, ldb, flags, p * panel::PNC);
+                panel::panel_zero<T>(Bp, k, nv, ldb, flags, p * panel::PNC, panel::PNC);
             else
-                panel::panel_solve<T>(Ap, Bp, k, nv, lda, ldb, flags, alpha, p * panel::PNC,
-                                      vb_smem);
+            {
+                panel::PanelSolver<T, 4, 1, true> s;
+                s.run(Ap, Bp, k, nv, lda, ldb, flags, alpha, p * panel::PNC, vb_smem, pw);
+            }
         }
     }
 }
@@ -216,18 +218,13 @@ rocblas_status vbatched_launch(rocblas_handle h, VbArgs<T> a)
     rocblas_status st = launch_status();
     if(st != rocblas_status_success)
         return st;
-    const size_t lds = panel::lds_bytes<T>(kPanelMaxK);
-    static const hipError_t opt = hipFuncSetAttribute(
-        reinterpret_cast<const void*>(&vb_panel_kernel<T>),
-        hipFuncAttributeMaxDynamicSharedMemorySize, int(lds));
-    (void)opt;
-    (void)hipGetLastError();
     int gmax = 1;
     for(int b = 0; b < kVbPanelBuckets; ++b)
         gmax = std::max(gmax, a.groups[b]);
     const int wgs = int(std::min<int64_t>(int64_t(a.batch) * gmax,
                                           int64_t(h->num_cus) * g_vb_tuning.panel_wgs_per_cu));
-    hipLaunchKernelGGL(vb_panel_kernel<T>, dim3(wgs), dim3(panel::PNT), lds, h->stream, a);
+    hipLaunchKernelGGL(vb_panel_kernel<T>, dim3(wgs), dim3(panel::PNT), 0, h->stream, a,
+                       panel::panel_wait(h));
     return launch_status();
 }
 
