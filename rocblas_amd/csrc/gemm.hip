@@ -13,6 +13,7 @@
 // diagonal block; such products with few tiles split their tiles' K ranges or
 // balance their K steps over the workgroups.
 #include "device_common.hpp"
+#include "gemm_tile.hpp"
 
 #include <cstdlib>
 #include <type_traits>
@@ -1418,7 +1419,21 @@ static rocblas_status launch_gemm_sel(rocblas_handle h, const GemmArgsT<TA, TB, 
            && tiles(128, 128) < 2 * cus && gemm_dma_eligible(a, 8))
             return launch_gemm_dma_split(h, a);
     }
-    if(tiles(128, 128) >= cus)
+    // Dense products with few 128 x 128 tiles run on smaller ones
+    // (gemm_tile.hip), which fill the last wave of workgroups better: below
+    // four per CU with 16-byte loads, below two with the 4-byte loads of
+    // unaligned operands, whose issue rate a 128 x 128 tile halves.  Measured
+    // on MI355X, TF/s of 128 x 128 / 64 x 64 tiles: FP64 256 x 16384 x 256 (256
+    // tiles) 37.8 / 49.8, 2048^3 (256) 56.9 / 66.4, 512 x 16384 x 512 (512)
+    // 55.6 / 61.3, unaligned 2048 x 4096 x 2048 (512) 66.7 / 51.3; FP32
+    // unaligned 1465 x 2999 x 1536 (288) 62 / 80.
+    int64_t few = cus;
+    if constexpr(std::is_same_v<TA, TB> && std::is_same_v<TA, TC>)
+    {
+        if(gemm_dma_mode() && gemm_tile_eligible(a))
+            few = gemm_tile_vec16(a) ? 4 * cus : 2 * cus;
+    }
+    if(tiles(128, 128) >= few)
     {
         // FP64 runs best with K steps of 8 (two waves per SIMD), FP32 with 16
         // (measured at 8192x16384x8192 on MI355X: 65 vs 50 TF/s, 96 vs 94 TF/s)
@@ -1453,10 +1468,20 @@ static rocblas_status launch_gemm_sel(rocblas_handle h, const GemmArgsT<TA, TB, 
                 return launch_status();
             }
         }
+        if constexpr(std::is_same_v<TA, TB> && std::is_same_v<TA, TC>)
+        {
+            if(gemm_dma_mode() && gemm_tile_eligible(a) && a.K % (128 / int(sizeof(TA))) == 0)
+                return launch_gemm_tile(h, a, 128);
+        }
         if constexpr(std::is_same_v<mfma_t<TA, TB>, double>)
             return launch_gemm_cfg<TA, TB, TC, 128, 128, 8, 2, 2>(h, a);
         else
             return launch_gemm_cfg<TA, TB, TC, 128, 128, 16, 2, 2>(h, a);
+    }
+    if constexpr(std::is_same_v<TA, TB> && std::is_same_v<TA, TC>)
+    {
+        if(gemm_dma_mode() && gemm_tile_eligible(a))
+            return launch_gemm_tile(h, a, tiles(64, 64) >= cus ? 64 : 32);
     }
     if(tiles(64, 64) >= cus)
         return launch_gemm_cfg<TA, TB, TC, 64, 64, 16, 2, 2>(h, a);
