@@ -178,7 +178,7 @@ inline unsigned grid_batch(int batch)
 }
 
 // ---------------------------------------------------------------------------
-// Small solve (k <= 64)
+// Small solve (k <= 32), and the arguments the panel and chained solves share
 // ---------------------------------------------------------------------------
 enum SmallFlags : int
 {
@@ -188,8 +188,7 @@ enum SmallFlags : int
     SF_UNIT  = 8,  // unit diagonal: the diagonal of A is never read
     SF_COLS  = 16, // the vectors are columns of B (side left)
     SF_SCALE = 32, // multiply the right-hand side by alpha
-    SF_DPP   = 64, // register-resident triangles with DPP row broadcasts (KMAX <= 32)
-    SF_FULL  = 128 // DPP launch with K == KMAX and every slot holding 16 vectors
+    SF_FULL  = 64  // small-solve launch with K == KMAX and every slot holding 16 vectors
 };
 
 template <typename T>
@@ -201,40 +200,20 @@ struct SmallArgs
     int               nvec;
     int               lda;
     int               ldb;
-    int               vp_log2;     // vectors per slot = 1 << vp_log2
-    int               chunks;      // ceil(nvec / vectors per slot)
-    int64_t           units;       // batch * chunks
+    int               chunks;    // ceil(nvec / vectors per slot)
+    int64_t           units;     // batch * chunks
     int               flags;
-    int               slot_stride; // elements per slot of the packed triangle in LDS
-    int               bs_stride;   // elements per staged vector (side L)
+    int               bs_stride; // elements per staged vector (side L)
     T                 alpha_host;
     const T*          alpha_dev;
 };
 
-// Largest number of instance slots per wavefront of the LDS variant for a
-// given KMAX: keeps the triangles' LDS region near 17-19 KiB.
-constexpr int small_gmax(int kmax)
-{
-    return kmax <= 8 ? 64 : kmax <= 16 ? 16 : kmax <= 32 ? 4 : kmax <= 48 ? 2 : 1;
-}
+constexpr int DPP_VP = 16; // vectors per slot of the small solve
+constexpr int DPP_G  = 4;  // slots per wavefront
 
-// packed canonical lower layout: element (i, j), i >= j, at colstart(j) + i - j
-template <int KMAX>
-__host__ __device__ constexpr int colstart(int j)
-{
-    return j * KMAX - j * (j - 1) / 2;
-}
-
-constexpr int slot_elems(int kmax)
-{
-    // odd, so consecutive slots start in different LDS banks
-    return (kmax * (kmax + 1) / 2) | 1;
-}
-
-// Single-launch panel solve for k <= kPanelMaxK (panel_trsm.hip; below 64 only
-// where the driver prefers it to the small kernels):
-// one workgroup per 16 vectors, same SmallArgs (K, nvec, lda, ldb, flags,
-// alpha); `units` is ignored (the batch count is passed separately).
+// Single-launch panel solve for k <= kPanelMaxK (panel_trsm.hip): one workgroup
+// per 16 or 32 vectors, same SmallArgs (K, nvec, lda, ldb, flags, alpha);
+// `units` is ignored (the batch count is passed separately).
 constexpr int kPanelMaxK = 512;
 
 template <typename T>

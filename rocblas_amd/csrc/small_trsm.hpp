@@ -1,4 +1,4 @@
-// small_trsm.hpp -- the k <= 64 triangular-solve kernel (instantiated per KMAX
+// small_trsm.hpp -- the k <= 32 triangular-solve kernel (instantiated per KMAX
 // in small_k*.hip).
 //
 // Every side/uplo/trans case is reduced to forward substitution L y = c on a
@@ -11,20 +11,15 @@
 // The matrix is embedded in a KMAX x KMAX triangle: entries outside the K x K
 // problem are 0 (1 on the diagonal) and right-hand-side entries outside it are
 // 0, so padded rows never change real rows -- and because the reversal is
-// relative to KMAX, every LDS offset in the substitution is a compile-time
+// relative to KMAX, every offset in the substitution is a compile-time
 // constant for each (UPPER, TA) variant.
 //
-// A wavefront serves G "slots" (instances) of VP vectors each (G * VP = 64).
-// Data movement, designed for one HBM round trip per wavefront:
-//   1. issue every global load: right-hand sides (side L: coalesced down the
-//      columns, staged through LDS so lane v can read column v; side R: one
-//      row per lane, already coalesced across lanes), then the slots' stored
-//      triangles in pair order (below);
-//   2. write the triangles to LDS in that same stored order (no index
-//      transform), diagonal replaced by its reciprocal;
-//   3. fully unrolled substitution; L[i][j] is read (LDS broadcast within a
-//      slot) from the stored position of A's entry;
-//   4. side L: solutions staged through LDS again for coalesced stores.
+// A wavefront serves four slots (instances) of 16 vectors each, also where an
+// instance has fewer vectors: packing more, narrower slots with the triangles
+// in LDS measured slower at every size (FP64, side L, 20000 instances of
+// order 32 with 8 vectors 102 us against 40, order 8 with one vector 11.8
+// against 5.9; one instance of order 32 with 8 vectors 17.4 against 8.6).
+// Every global load of a wavefront is issued before the first wait.
 //
 // Pair order: within a KMAX x KMAX triangle, column c and column KMAX-1-c
 // together hold exactly KMAX+1 entries, so entry t lies in pair t / (KMAX+1)
@@ -35,23 +30,6 @@
 
 namespace rbamd
 {
-
-// Returns v unchanged through an empty asm, so comparisons against the result
-// are recomputed where they are used instead of being hoisted and kept live
-// (dozens of live per-row masks otherwise spill the scalar registers).
-__device__ __forceinline__ int fresh(int v)
-{
-    asm volatile("" : "+s"(v));
-    return v;
-}
-
-// Same for a per-lane value: address arithmetic derived from the result is
-// recomputed instead of being shared with (and kept live from) earlier phases.
-__device__ __forceinline__ int fresh_lane(int v)
-{
-    asm volatile("" : "+v"(v));
-    return v;
-}
 
 // offset of stored entry (p, q) of a KMAX triangle in pair order
 template <int KMAX, bool UPPER>
@@ -85,7 +63,7 @@ __host__ __device__ inline void pair_decode(int t, int& p, int& q)
     }
 }
 
-// LDS offset of canonical L[i][j]
+// pair-order offset of canonical L[i][j]
 template <int KMAX, bool UPPER, bool TA>
 __host__ __device__ constexpr int lofs(int i, int j)
 {
@@ -96,224 +74,7 @@ __host__ __device__ constexpr int lofs(int i, int j)
 }
 
 // ---------------------------------------------------------------------------
-// LDS variant (any KMAX, any vectors-per-slot): the slots' triangles live in
-// LDS in stored pair order and every lane reads L[i][j] as an LDS broadcast.
-// Region layout: [G slots x slot_stride] triangles, then (side L) the
-// 64 x bs_stride staging area for the right-hand sides.
-// ---------------------------------------------------------------------------
-template <typename T, int KMAX, bool UPPER, bool TA, bool COLS>
-__global__ void __launch_bounds__(WAVE) small_trsm_lds_kernel(const SmallArgs<T> a)
-{
-    constexpr bool REV     = UPPER != TA;
-    constexpr int  TRI     = KMAX * (KMAX + 1) / 2;
-    constexpr int  BATCHLD = 16;
-
-    extern __shared__ __align__(16) unsigned char smem_raw[];
-    T* const R = reinterpret_cast<T*>(smem_raw);
-    __shared__ const T* slotA[WAVE];
-    __shared__ T*       slotB[WAVE];
-    __shared__ int      slotV0[WAVE];
-
-    const int  lane  = threadIdx.x;
-    const int  vpl   = a.vp_log2;
-    const int  VP    = 1 << vpl;
-    const int  G     = WAVE >> vpl;
-    const int  g     = lane >> vpl;
-    const int  v     = lane & (VP - 1);
-    const int  K     = a.K;
-    const bool unit  = a.flags & SF_UNIT;
-    const bool scale = a.flags & SF_SCALE;
-    const int  lda   = a.lda;
-    const int  ldb   = a.ldb;
-    const int  bs    = a.bs_stride;
-    const int  S     = a.slot_stride;
-    T* const   RB    = R + G * S; // side-L staging area
-
-    const T alpha = a.alpha_dev ? *a.alpha_dev : a.alpha_host;
-
-    if(lane < G)
-    {
-        const int64_t u = int64_t(blockIdx.x) * G + lane;
-        if(u < a.units)
-        {
-            const int64_t inst = a.chunks == 1 ? u : u / a.chunks;
-            slotA[lane]        = a.A.get(inst);
-            slotB[lane]        = a.B.get(inst);
-            slotV0[lane]       = int(u - inst * a.chunks) * VP;
-        }
-        else
-        {
-            slotA[lane]  = nullptr;
-            slotB[lane]  = nullptr;
-            slotV0[lane] = 0;
-        }
-    }
-    __syncthreads();
-
-    T* const   myB   = slotB[g];
-    const int  vec   = slotV0[g] + v;
-    const bool valid = myB != nullptr && vec < a.nvec;
-
-    if(alpha == T(0))
-    {
-        // B := 0 and A is not referenced (uniform branch: alpha is global)
-        if(valid)
-            for(int i = 0; i < K; ++i)
-                gstore(myB + (COLS ? (i + int64_t(vec) * ldb) : (vec + int64_t(i) * ldb)), T(0));
-        return;
-    }
-
-    // Out-of-range lanes load from a valid address (slot 0 always exists) and
-    // discard the value, so no load sits behind a branch.
-    const T* const safeA = slotA[0];
-    T* const       safeB = slotB[0];
-
-    // ---- 1. right-hand sides -> staging area (lane v later reads vector v) ----
-    // side L: coalesced down the columns; side R: lane v loads row v (already
-    // coalesced across lanes).  Parking the values in LDS keeps them out of
-    // registers while the triangles are loaded.
-    T c[KMAX];
-    for(int s0 = 0; s0 < KMAX; s0 += BATCHLD)
-    {
-        T   bv[BATCHLD];
-        int Kc = fresh(K);
-#pragma unroll
-        for(int s = 0; s < BATCHLD; ++s)
-        {
-            if constexpr(COLS)
-            {
-                const int  e  = lane + WAVE * (s0 + s);
-                const int  r  = e % KMAX;
-                const int  v2 = e / KMAX;
-                T* const   Bp = slotB[v2 >> vpl];
-                const int  vc = slotV0[v2 >> vpl] + (v2 & (VP - 1));
-                const bool ok = s0 + s < KMAX && Bp && r < Kc && vc < a.nvec;
-                const T    x  = gload(ok ? Bp + (r + int64_t(vc) * ldb) : safeB);
-                bv[s]         = ok ? x : T(0);
-            }
-            else
-            {
-                const int  r  = s0 + s;
-                const bool ok = valid && r < Kc;
-                const T    x  = gload(ok ? myB + (vec + int64_t(r) * ldb) : safeB);
-                bv[s]         = ok ? x : T(0);
-            }
-        }
-#pragma unroll
-        for(int s = 0; s < BATCHLD; ++s)
-        {
-            if(s0 + s < KMAX)
-            {
-                if constexpr(COLS)
-                {
-                    const int e  = lane + WAVE * (s0 + s);
-                    const int r  = e % KMAX;
-                    const int v2 = e / KMAX;
-                    RB[v2 * bs + (REV ? KMAX - 1 - r : r)] = bv[s];
-                }
-                else
-                {
-                    const int r = s0 + s;
-                    RB[lane * bs + (REV ? KMAX - 1 - r : r)] = bv[s];
-                }
-            }
-        }
-    }
-
-    // ---- 2. triangles -> LDS in stored pair order ----
-    const int totalA = G * TRI;
-    for(int t0 = 0; t0 < totalA; t0 += WAVE * BATCHLD)
-    {
-        T av[BATCHLD];
-#pragma unroll
-        for(int s = 0; s < BATCHLD; ++s)
-        {
-            const int e  = t0 + lane + WAVE * s;
-            const int g2 = e / TRI;
-            int       p, q;
-            pair_decode<KMAX, UPPER>(e % TRI, p, q);
-            const T*   Ap   = e < totalA ? slotA[g2] : nullptr;
-            const bool load = Ap && p < K && q < K && !(unit && p == q);
-            const T    x    = gload(load ? Ap + (p + int64_t(q) * lda) : safeA);
-            av[s]           = load ? x : (p == q ? T(1) : T(0));
-        }
-#pragma unroll
-        for(int s = 0; s < BATCHLD; ++s)
-        {
-            const int e = t0 + lane + WAVE * s;
-            if(e < totalA)
-                R[(e / TRI) * S + e % TRI] = av[s];
-        }
-    }
-    __syncthreads();
-#pragma unroll
-    for(int i = 0; i < KMAX; ++i)
-        c[i] = RB[lane * bs + i];
-    if(!unit)
-    {
-        for(int idx = lane; idx < G * KMAX; idx += WAVE)
-        {
-            const int j = idx % KMAX;
-            T&        d = R[(idx / KMAX) * S + pair_off<KMAX, UPPER>(j, j)];
-            d           = T(1) / d;
-        }
-        __syncthreads();
-    }
-    if(scale)
-    {
-#pragma unroll
-        for(int i = 0; i < KMAX; ++i)
-            c[i] *= alpha;
-    }
-
-    // ---- 3. forward substitution on the canonical lower triangle ----
-    const T* L = R + g * S;
-#pragma unroll
-    for(int j = 0; j < KMAX; ++j)
-    {
-        const T x = c[j] * L[lofs<KMAX, UPPER, TA>(j, j)];
-        c[j]      = x;
-#pragma unroll
-        for(int i = j + 1; i < KMAX; ++i)
-            c[i] = fma(-L[lofs<KMAX, UPPER, TA>(i, j)], x, c[i]);
-        // bound how far ahead the scheduler hoists LDS reads (registers)
-        if(KMAX > 32 || j % 2 == 1)
-            asm volatile("" ::: "memory");
-    }
-
-    // ---- 4. store: solutions staged through LDS again ----
-    // side L: coalesced down the columns; side R: lane v stores row v.
-#pragma unroll
-    for(int i = 0; i < KMAX; ++i)
-        RB[lane * bs + i] = c[i];
-    __syncthreads();
-    int       Kc = fresh(K);
-    const int ln = fresh_lane(lane);
-#pragma unroll
-    for(int s = 0; s < KMAX; ++s)
-    {
-        if(s % 8 == 0)
-            Kc = fresh(Kc);
-        if constexpr(COLS)
-        {
-            const int e  = ln + WAVE * s;
-            const int r  = e % KMAX;
-            const int v2 = e / KMAX;
-            T* const  Bp = slotB[v2 >> vpl];
-            const int vc = slotV0[v2 >> vpl] + (v2 & (VP - 1));
-            if(Bp && r < Kc && vc < a.nvec)
-                gstore(Bp + (r + int64_t(vc) * ldb), RB[v2 * bs + (REV ? KMAX - 1 - r : r)]);
-        }
-        else
-        {
-            if(valid && s < Kc)
-                gstore(myB + (vec + int64_t(s) * ldb), RB[lane * bs + (REV ? KMAX - 1 - s : s)]);
-        }
-    }
-}
-
-// ---------------------------------------------------------------------------
-// DPP variant (KMAX <= 32; slots of 16 vectors, four slots per wavefront):
+// The kernel (KMAX <= 32; slots of 16 vectors, four slots per wavefront):
 // each 16-lane row holds its slot's triangle in registers -- entry t of the
 // pair order in lane t % 16, register t / 16, stored negated -- and every
 // update c[i] -= L[i][j] x_j is a single v_fmac_{f64,f32}_dpp whose first
@@ -330,8 +91,6 @@ __global__ void __launch_bounds__(WAVE) small_trsm_lds_kernel(const SmallArgs<T>
 // constant plus a uniform base.  FULL launches (K == KMAX, every slot holds
 // 16 vectors) carry no masks at all.
 // ---------------------------------------------------------------------------
-constexpr int DPP_VP = 16; // vectors per slot
-constexpr int DPP_G  = 4;  // slots per wavefront
 
 template <typename T, int KMAX>
 using DppTri = T[(KMAX * (KMAX + 1) / 2 + 15) / 16];
@@ -603,24 +362,10 @@ template <typename T, int KMAX, bool UPPER, bool TA>
 static rocblas_status launch_small_side(rocblas_handle h, const SmallArgs<T>& a, dim3 grid,
                                         size_t lds)
 {
-    const bool cols = a.flags & SF_COLS;
-    if constexpr(KMAX <= 32)
-    {
-        if(a.flags & SF_DPP)
-        {
-            if(cols)
-                launch_dpp<T, KMAX, UPPER, TA, true>(h, a, grid, lds);
-            else
-                launch_dpp<T, KMAX, UPPER, TA, false>(h, a, grid, lds);
-            return launch_status();
-        }
-    }
-    if(cols)
-        hipLaunchKernelGGL((small_trsm_lds_kernel<T, KMAX, UPPER, TA, true>), grid, dim3(WAVE),
-                           lds, h->stream, a);
+    if(a.flags & SF_COLS)
+        launch_dpp<T, KMAX, UPPER, TA, true>(h, a, grid, lds);
     else
-        hipLaunchKernelGGL((small_trsm_lds_kernel<T, KMAX, UPPER, TA, false>), grid, dim3(WAVE),
-                           lds, h->stream, a);
+        launch_dpp<T, KMAX, UPPER, TA, false>(h, a, grid, lds);
     return launch_status();
 }
 

@@ -1,13 +1,15 @@
 // trsm_driver.hip -- dispatch of rocblas_?trsm onto the gfx950 kernels.
 //
-//   k <= 64: one launch of the small substitution kernel (small_trsm.hpp),
-//            all instances and right-hand sides of the call in one grid.
-//   k >  64: recursive blocked solve on the canonical index range (the
+//   k <= 32: one launch of the small substitution kernel (small_trsm.hpp),
+//            all instances and right-hand sides of the call in one grid;
+//   k <= 512: one launch of the panel solve (panel_trsm.hpp);
+//   longer, one instance, few vectors: one chained launch (chain_trsm.hip);
+//   else: recursive blocked solve on the canonical index range (the
 //            reduction of every side/uplo/trans case to forward substitution
 //            on L = P M P is described in small_trsm.hpp):
 //              y1 = solve(L11, c1);  c2 -= L21 y1 (MFMA GEMM, gemm.hip);
 //              y2 = solve(L22, c2)
-//            with leaves of at most 64 solved in place by the small kernel.
+//            with leaves solved in place by the panel solve.
 //            The GEMM updates at the top of the recursion are large and
 //            square-ish, which is where almost all of the m*n*k flops are.
 //
@@ -144,109 +146,41 @@ template rocblas_status copy_launch<double>(rocblas_handle, int, int, BatchPtr<c
 // ---------------------------------------------------------------------------
 // Small-solve launch plan
 // ---------------------------------------------------------------------------
-struct SmallPlan
-{
-    int    kmax;
-    int    vp_log2;
-    int    G;
-    int    slot_stride;
-    int    bs_stride;
-    size_t lds_elems;
-    size_t lds_bytes;
-};
-
-// Two kernel variants (small_trsm.hpp):
-//   DPP  (KMAX <= 32 and more than 8 vectors per instance): four slots of
-//        16 vectors per wavefront, triangles in registers; LDS only stages
-//        side-L right-hand sides.
-//   LDS  (otherwise): VP = next power of two >= nvec, G = 64 / VP slots per
-//        wavefront capped by small_gmax(KMAX) (by widening the slots);
-//        triangles in LDS.
-template <typename T>
-static SmallPlan plan_small(int K, int nvec, bool cols, bool& dpp)
-{
-    SmallPlan s;
-    s.kmax        = K <= 8 ? 8 : K <= 16 ? 16 : K <= 32 ? 32 : K <= 48 ? 48 : 64;
-    s.slot_stride = slot_elems(s.kmax);
-    s.bs_stride   = s.kmax + 1;
-    dpp           = s.kmax <= 32 && nvec > 8;
-    int vp        = 1;
-    while(vp < std::min(nvec, WAVE))
-        vp <<= 1;
-    if(dpp)
-        vp = 16;
-    int G = WAVE / vp;
-    while(!dpp && G > small_gmax(s.kmax))
-    {
-        G >>= 1;
-        vp <<= 1;
-    }
-    s.G       = G;
-    s.vp_log2 = 0;
-    while((1 << s.vp_log2) < vp)
-        ++s.vp_log2;
-    // staging: side L for the DPP variant, both sides for the LDS variant
-    const size_t staging = (cols || !dpp) ? size_t(WAVE) * s.bs_stride : 0;
-    s.lds_elems          = (dpp ? 0 : size_t(G) * s.slot_stride) + staging;
-    s.lds_bytes          = s.lds_elems * sizeof(T);
-    return s;
-}
+// k <= kSmallMaxK: four slots of 16 vectors per wavefront (small_trsm.hpp).
+constexpr int kSmallMaxK = 32;
 
 template <typename T>
 static rocblas_status launch_small(rocblas_handle h, const SmallArgs<T>& args_in, int batch)
 {
-    SmallArgs<T>    a    = args_in;
-    const bool      cols = a.flags & SF_COLS;
-    bool            dpp  = false;
-    const SmallPlan s    = plan_small<T>(a.K, a.nvec, cols, dpp);
-    if(dpp)
-        a.flags |= SF_DPP;
-    const int       VP   = 1 << s.vp_log2;
-    a.vp_log2            = s.vp_log2;
-    a.chunks             = (a.nvec + VP - 1) / VP;
+    SmallArgs<T> a       = args_in;
+    const bool   cols    = a.flags & SF_COLS;
+    const int    kmax    = a.K <= 8 ? 8 : a.K <= 16 ? 16 : 32;
+    a.chunks             = (a.nvec + DPP_VP - 1) / DPP_VP;
     a.units              = int64_t(batch) * a.chunks;
-    a.slot_stride        = s.slot_stride;
-    a.bs_stride          = s.bs_stride;
-    if(dpp && a.K == s.kmax && a.nvec % VP == 0 && a.units % s.G == 0)
+    a.bs_stride          = kmax + 1;
+    const size_t lds     = cols ? size_t(WAVE) * a.bs_stride * sizeof(T) : 0; // staging
+    if(a.K == kmax && a.nvec % DPP_VP == 0 && a.units % DPP_G == 0)
         a.flags |= SF_FULL;
-    const int64_t blocks = (a.units + s.G - 1) / s.G;
+    const int64_t blocks = (a.units + DPP_G - 1) / DPP_G;
     if(blocks > int64_t(0x7fffffff))
         return rocblas_status_invalid_size;
     const dim3 grid{unsigned(blocks)};
-    switch(s.kmax)
+    switch(kmax)
     {
     case 8:
-        return launch_small_kmax<T, 8>(h, a, grid, s.lds_bytes);
+        return launch_small_kmax<T, 8>(h, a, grid, lds);
     case 16:
-        return launch_small_kmax<T, 16>(h, a, grid, s.lds_bytes);
-    case 32:
-        return launch_small_kmax<T, 32>(h, a, grid, s.lds_bytes);
-    case 48:
-        return launch_small_kmax<T, 48>(h, a, grid, s.lds_bytes);
+        return launch_small_kmax<T, 16>(h, a, grid, lds);
     default:
-        return launch_small_kmax<T, 64>(h, a, grid, s.lds_bytes);
+        return launch_small_kmax<T, 32>(h, a, grid, lds);
     }
 }
 
 // ---------------------------------------------------------------------------
 // Driver
 // ---------------------------------------------------------------------------
-constexpr int SMALL_K = 64; // largest k solved by the small kernel / leaf size
+constexpr int SMALL_K = 64; // granularity of the recursion's splits
 
-// A solve with k <= SMALL_K takes the small kernels (triangle in registers or
-// in one wavefront's LDS) except where the panel solve is as fast or faster:
-// 48 < k, or 32 < k with at most 16 vectors.  Measured on MI355X, side L,
-// strided batch of 20000 (small kernels / panel kernel behind the variable-
-// size batch's planning launch):
-//   k = 64, n = 16: 1000 / 416 us;  k = 48, n = 16: 380 / 377 us;
-//   k = 64, n = 64: 1076 / 1097 us; k = 48, n = 64: 548 / 1027 us;
-//   one instance, k = 64, n = 16: 38 / 17 us; k = 64, n = 64: 39 / 31 us.
-// The choice depends on k and the vector count only, so a batched solve and
-// the single solves of its instances take the same kernels (and bits).
-inline bool small_kernel_preferred(int K, int nvec)
-{
-    return K <= 32 || (K <= 48 && nvec > 16);
-}
 // leaves of the recursion for right-hand sides of at least kWidePanels panels
 constexpr int kWideLeafK  = 256;
 constexpr int kWidePanels = 64;
@@ -331,7 +265,7 @@ struct Solver
         return launch_gemm(h, g);
     }
 
-    // SMALL_K < k <= kPanelMaxK: one launch solves the whole range
+    // kSmallMaxK < k <= kPanelMaxK: one launch solves the whole range
     rocblas_status panel_leaf(int a, int b)
     {
         const int    K  = b - a;
@@ -353,7 +287,7 @@ struct Solver
     rocblas_status solve(int a, int b)
     {
         const int K = b - a;
-        if(K <= SMALL_K)
+        if(K <= kSmallMaxK)
             return leaf(a, b);
         // A panel leaf streams its whole triangle once per 16-vector panel;
         // with many panels the work is better spent in GEMM updates, so wide
@@ -394,7 +328,12 @@ rocblas_status trsm_launch(rocblas_handle h, const TrsmProblem<T>& p)
     const bool  lowerM = (!upperA) != tA;
     const int   K      = sideL ? p.m : p.n;
 
-    if(K <= SMALL_K && small_kernel_preferred(K, sideL ? p.n : p.m))
+    // The choice depends on k only, so a batched solve and the single solves
+    // of its instances take the same kernels (and bits).  Triangles of 33 to 64
+    // rows take the panel solve: FP64, side L, against one wavefront walking
+    // the triangle through LDS, k = 48 with 64 vectors 25 -> 5.0 us alone and
+    // 545 -> 355 us for 20000 instances.
+    if(K <= kSmallMaxK)
     {
         SmallArgs<T> s{};
         s.A          = p.A;

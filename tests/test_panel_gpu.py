@@ -49,7 +49,7 @@ CASES = [("L", "L", "N"), ("L", "U", "N"), ("L", "L", "T"), ("R", "U", "N"), ("R
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("prec", ["d", "s"])
-@pytest.mark.parametrize("k", [49, 64, 65, 80, 113, 255, 256, 257, 272, 511, 512])
+@pytest.mark.parametrize("k", [33, 49, 64, 65, 80, 113, 255, 256, 257, 272, 511, 512])
 def test_edges_against_oracle_one_and_batched(h, k, prec):
     rng = np.random.default_rng(k)
     for i, (side, uplo, trans) in enumerate(CASES):
