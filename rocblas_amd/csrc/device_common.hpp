@@ -222,11 +222,10 @@ bool panel_fits(rocblas_handle h, int K);
 template <typename T>
 rocblas_status launch_panel(rocblas_handle h, const SmallArgs<T>& a, int batch);
 
-// Chained single-instance solve (chain_trsm.hip): one workgroup per (64-row
-// block, 16-vector panel), blocks chained through per-panel completion
-// counters in the handle's chain_flags buffer (kChainFlagsBytes: one 64-bit
-// counter per panel, then an error word).
-constexpr int kChainMaxPanels = int(kChainFlagsBytes / 8) - 1;
+// Chained single-instance solve (chain_trsm.hip): one workgroup per (super-
+// block of rows, 16-vector panel), handing the solution on through B and per-
+// panel flags in the handle's chain_flags buffer (32 bytes per panel).
+constexpr int kChainMaxPanels = int(kChainFlagsBytes / 32);
 
 template <typename T>
 bool chain_fits(rocblas_handle h, int K, int nvec, int batch);

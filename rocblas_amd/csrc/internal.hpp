@@ -40,7 +40,7 @@ struct _rocblas_handle
     bool                 ws_in_use     = false;
     bool                 size_query    = false;
     size_t               query_size    = 0;
-    // completion counters of the chained solve (chain_trsm.hip): one per
+    // flags of the chained solve (chain_trsm.hip): eight words per
     // panel, zero between launches; followed in the same allocation by the
     // tile counters of the split-K GEMM (kSplitCounters, zero between launches)
     void*                chain_flags   = nullptr;
@@ -60,8 +60,8 @@ struct _rocblas_handle
 
 namespace rbamd
 {
-// Bytes of a handle's chain_flags buffer.
-constexpr size_t kChainFlagsBytes = 4096;
+// Bytes of a handle's chain_flags buffer: 32 per vector panel.
+constexpr size_t kChainFlagsBytes = 16384;
 // Tile counters of the split-K GEMM after them: one per (instance, tile) of a
 // split launch.
 constexpr int kSplitCounters = 4096;

@@ -27,8 +27,8 @@ __device__ __forceinline__ void panel_unit(const SmallArgs<T>& a, panel::PanelWa
         panel::panel_zero<T>(Bp, a.K, a.nvec, a.ldb, a.flags, v0, panel::PNC * NVG);
     else
     {
-        panel::PanelSolver<T, NT, NVG, false> s;
-        s.run(a.A.get(b), Bp, a.K, a.nvec, a.lda, a.ldb, a.flags, scale, v0, smem, pw);
+        panel::panel_solve<T, NT, NVG, panel::PM_SINGLE>(
+            a.A.get(b), Bp, a.K, a.nvec, a.lda, a.ldb, a.flags, scale, v0, smem, pw);
     }
 }
 

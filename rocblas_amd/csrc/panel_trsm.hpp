@@ -67,14 +67,15 @@ constexpr size_t lds_bytes()
     return sizeof(T) * PNC * (size_t(PRING) * NVG * ypitch<T>() + 4 * (ypitch<T>() + 1)) + 16;
 }
 
-// One substitution step for the four vectors a 16-lane row holds:
-// c_r += c_r[lane J] * l, with l = -L[g][J] / L[J][J] below the diagonal and 0
-// elsewhere.  A register is read through DPP four VALU instructions after the
-// previous step wrote it; the padding of step 0 covers whatever came before.
-template <int J>
+// One substitution step for the vectors a 16-lane row holds, one per register
+// r < NR: c_r += c_r[lane J] * l, with l = -L[g][J] / L[J][J] below the
+// diagonal and 0 elsewhere.  A register is read through DPP at least two wait
+// states after the previous step wrote it (the other registers' updates, or
+// padding); the padding of step 0 covers whatever came before.
+template <int J, int NR>
 __device__ __forceinline__ void solve_step(double (&c)[4], double l)
 {
-    if constexpr(J == 0)
+    if constexpr(NR == 4 && J == 0)
         asm volatile("s_nop 4\n\t"
                      "v_fmac_f64_dpp %0, %0, %4 row_newbcast:%5 row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t"
                      "v_fmac_f64_dpp %1, %1, %4 row_newbcast:%5 row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t"
@@ -82,19 +83,40 @@ __device__ __forceinline__ void solve_step(double (&c)[4], double l)
                      "v_fmac_f64_dpp %3, %3, %4 row_newbcast:%5 row_mask:0xf bank_mask:0xf bound_ctrl:1"
                      : "+v"(c[0]), "+v"(c[1]), "+v"(c[2]), "+v"(c[3])
                      : "v"(l), "n"(J));
-    else
+    else if constexpr(NR == 4)
         asm volatile("v_fmac_f64_dpp %0, %0, %4 row_newbcast:%5 row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t"
                      "v_fmac_f64_dpp %1, %1, %4 row_newbcast:%5 row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t"
                      "v_fmac_f64_dpp %2, %2, %4 row_newbcast:%5 row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t"
                      "v_fmac_f64_dpp %3, %3, %4 row_newbcast:%5 row_mask:0xf bank_mask:0xf bound_ctrl:1"
                      : "+v"(c[0]), "+v"(c[1]), "+v"(c[2]), "+v"(c[3])
                      : "v"(l), "n"(J));
+    if constexpr(NR == 2 && J == 0)
+        asm volatile("s_nop 4\n\t"
+                     "v_fmac_f64_dpp %0, %0, %2 row_newbcast:%3 row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t"
+                     "v_fmac_f64_dpp %1, %1, %2 row_newbcast:%3 row_mask:0xf bank_mask:0xf bound_ctrl:1"
+                     : "+v"(c[0]), "+v"(c[1])
+                     : "v"(l), "n"(J));
+    else if constexpr(NR == 2)
+        asm volatile("s_nop 0\n\t"
+                     "v_fmac_f64_dpp %0, %0, %2 row_newbcast:%3 row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t"
+                     "v_fmac_f64_dpp %1, %1, %2 row_newbcast:%3 row_mask:0xf bank_mask:0xf bound_ctrl:1"
+                     : "+v"(c[0]), "+v"(c[1])
+                     : "v"(l), "n"(J));
+    if constexpr(NR == 1 && J == 0)
+        asm volatile("s_nop 4\n\t"
+                     "v_fmac_f64_dpp %0, %0, %1 row_newbcast:%2 row_mask:0xf bank_mask:0xf bound_ctrl:1"
+                     : "+v"(c[0])
+                     : "v"(l), "n"(J));
+    else if constexpr(NR == 1)
+        asm volatile("s_nop 1\n\t"
+                     "v_fmac_f64_dpp %0, %0, %1 row_newbcast:%2 row_mask:0xf bank_mask:0xf bound_ctrl:1"
+                     : "+v"(c[0])
+                     : "v"(l), "n"(J));
 }
-
-template <int J>
+template <int J, int NR>
 __device__ __forceinline__ void solve_step(float (&c)[4], float l)
 {
-    if constexpr(J == 0)
+    if constexpr(NR == 4 && J == 0)
         asm volatile("s_nop 4\n\t"
                      "v_fmac_f32_dpp %0, %0, %4 row_newbcast:%5 row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t"
                      "v_fmac_f32_dpp %1, %1, %4 row_newbcast:%5 row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t"
@@ -102,16 +124,38 @@ __device__ __forceinline__ void solve_step(float (&c)[4], float l)
                      "v_fmac_f32_dpp %3, %3, %4 row_newbcast:%5 row_mask:0xf bank_mask:0xf bound_ctrl:1"
                      : "+v"(c[0]), "+v"(c[1]), "+v"(c[2]), "+v"(c[3])
                      : "v"(l), "n"(J));
-    else
+    else if constexpr(NR == 4)
         asm volatile("v_fmac_f32_dpp %0, %0, %4 row_newbcast:%5 row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t"
                      "v_fmac_f32_dpp %1, %1, %4 row_newbcast:%5 row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t"
                      "v_fmac_f32_dpp %2, %2, %4 row_newbcast:%5 row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t"
                      "v_fmac_f32_dpp %3, %3, %4 row_newbcast:%5 row_mask:0xf bank_mask:0xf bound_ctrl:1"
                      : "+v"(c[0]), "+v"(c[1]), "+v"(c[2]), "+v"(c[3])
                      : "v"(l), "n"(J));
+    if constexpr(NR == 2 && J == 0)
+        asm volatile("s_nop 4\n\t"
+                     "v_fmac_f32_dpp %0, %0, %2 row_newbcast:%3 row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t"
+                     "v_fmac_f32_dpp %1, %1, %2 row_newbcast:%3 row_mask:0xf bank_mask:0xf bound_ctrl:1"
+                     : "+v"(c[0]), "+v"(c[1])
+                     : "v"(l), "n"(J));
+    else if constexpr(NR == 2)
+        asm volatile("s_nop 0\n\t"
+                     "v_fmac_f32_dpp %0, %0, %2 row_newbcast:%3 row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t"
+                     "v_fmac_f32_dpp %1, %1, %2 row_newbcast:%3 row_mask:0xf bank_mask:0xf bound_ctrl:1"
+                     : "+v"(c[0]), "+v"(c[1])
+                     : "v"(l), "n"(J));
+    if constexpr(NR == 1 && J == 0)
+        asm volatile("s_nop 4\n\t"
+                     "v_fmac_f32_dpp %0, %0, %1 row_newbcast:%2 row_mask:0xf bank_mask:0xf bound_ctrl:1"
+                     : "+v"(c[0])
+                     : "v"(l), "n"(J));
+    else if constexpr(NR == 1)
+        asm volatile("s_nop 1\n\t"
+                     "v_fmac_f32_dpp %0, %0, %1 row_newbcast:%2 row_mask:0xf bank_mask:0xf bound_ctrl:1"
+                     : "+v"(c[0])
+                     : "v"(l), "n"(J));
 }
 
-template <typename T, int NVG, int J>
+template <typename T, int NVG, int NR, int J>
 struct SolveSteps
 {
     static __device__ __forceinline__ void run(T (&c)[NVG][4], const T (&l)[PNC - 1])
@@ -120,8 +164,8 @@ struct SolveSteps
         {
 #pragma unroll
             for(int v = 0; v < NVG; ++v)
-                solve_step<J>(c[v], l[J]);
-            SolveSteps<T, NVG, J + 1>::run(c, l);
+                solve_step<J, NR>(c[v], l[J]);
+            SolveSteps<T, NVG, NR, J + 1>::run(c, l);
         }
     }
 };
@@ -173,6 +217,22 @@ __device__ __forceinline__ void load4(T (&x)[4], const T* p)
     for(int r = 0; r < 4; ++r)
         x[r] = v[r];
 }
+// Agent-scope accesses: written through to, and read from, the point where the
+// XCDs' L2 caches agree
+template <typename T>
+__device__ __forceinline__ T coherent_load(const T* p)
+{
+    return __hip_atomic_load(const_cast<__attribute__((address_space(1))) T*>(
+                                 (const __attribute__((address_space(1))) T*)(p)),
+                             __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+template <typename T>
+__device__ __forceinline__ void coherent_store(T* p, T x)
+{
+    __hip_atomic_store((__attribute__((address_space(1))) T*)(p), x, __ATOMIC_RELAXED,
+                       __HIP_MEMORY_SCOPE_AGENT);
+}
+
 template <typename T>
 __device__ __forceinline__ void store4(T* p, const T (&x)[4])
 {
@@ -194,8 +254,23 @@ __device__ void panel_zero(T* Bp, int K, int nvec, int ldb, int flags, int v0, i
     }
 }
 
-// MULTI: K may exceed 64 NT rows (several super-blocks).
-template <typename T, int NT, int NVG, bool MULTI>
+// How a triangle of more than 64 NT rows is walked.
+enum PanelMode
+{
+    PM_SINGLE, // it has at most 64 NT rows: one super-block
+    PM_MULTI,  // this workgroup solves its super-blocks one after another
+    PM_CHAIN   // each super-block has a workgroup of its own (chain_trsm.hip)
+};
+
+// Flags of a panel of the chained solve, in device memory: word w counts the
+// sub-blocks of wavefront w (t % 4 == w, over all super-blocks) whose solution
+// is in B, word 4 the workgroups that have finished.
+constexpr int CHAIN_WORDS = 8;
+
+// NR: registers (vectors per 16-lane row) in use, 4 NR vectors of the group
+// KC: the columns of canonical L are contiguous in memory (op(A) transposed on
+// the left, plain on the right), so a lane's four operand entries are one load
+template <typename T, int NT, int NVG, PanelMode MODE, int NR, bool KC>
 struct PanelSolver
 {
     using acc_t             = typename Mfma<T>::acc_t;
@@ -219,12 +294,18 @@ struct PanelSolver
     // wavefront and lane
     int     w, g, q;
     int64_t lq; // 4 q columns
+    // operand kk is column 4 q + (kk ^ kx) of L: 3 where the columns run
+    // backwards in memory (KC, reversed), so that the load stays one ascending
+    // access; bk: the matching step between rows of B
+    int kx, bk;
     // LDS
     T*        Y;
     T*        D; // this wavefront's diagonal block and reciprocal diagonal
     int*      done;
     int       seen;
     PanelWait pw;
+    unsigned* link;  // PM_CHAIN: the panel's flags
+    int       avail; // PM_CHAIN: sub-blocks known to be in B
 
     // state: -sum of L y so far, L operands in flight; of the next sub-block to
     // solve the right-hand sides and the diagonal block
@@ -248,6 +329,19 @@ struct PanelSolver
         asm volatile("" : "+v"(p));
     }
 
+    // Vector of a group in register r of 16-lane group q: the result layout's
+    // order, except where only NR registers are used, which then hold the
+    // first 4 NR vectors in both types.
+    static __device__ __forceinline__ int group_vec(int q_, int r)
+    {
+        return NR == 4 ? mfma_row<T>(q_, r) : q_ + 4 * r;
+    }
+    // the same for an MFMA row (lane index l % 16 of the y operand)
+    static __device__ __forceinline__ int row_vec(int row)
+    {
+        return NR == 4 || sizeof(T) == 8 ? row : (row >> 2) + 4 * (row & 3);
+    }
+
     // operand registers of L(t, ev): row 16 t + g, columns 16 ev + 4 q + kk.
     // Rows past K - 1 (last sub-block) read row K - 1; they feed only rows
     // that are never stored.  ev < t, so every column is below K.
@@ -255,12 +349,17 @@ struct PanelSolver
     {
         const int row = min(PNC * t + g, K - 1);
         const T*  p   = Ab + int64_t(PNC * ev) * cs + (int64_t(row) * rs + lq);
-#pragma unroll
-        for(int kk = 0; kk < 4; ++kk)
+        if constexpr(KC)
+            load4(f, p);
+        else
         {
-            f[kk] = gload(p);
-            p += cs;
-            pin(p);
+#pragma unroll
+            for(int kk = 0; kk < 4; ++kk)
+            {
+                f[kk] = gload(p);
+                p += cs;
+                pin(p);
+            }
         }
     }
 
@@ -335,7 +434,7 @@ struct PanelSolver
     __device__ __forceinline__ void load_rhs(int t)
     {
         const T* p = Bb + int64_t(min(PNC * t + g, K - 1)) * br;
-        if(WIDE && full_rows)
+        if(WIDE && NR == 4 && MODE != PM_CHAIN && full_rows)
         {
 #pragma unroll
             for(int v = 0; v < NVG; ++v)
@@ -346,9 +445,8 @@ struct PanelSolver
 #pragma unroll
             for(int v = 0; v < NVG; ++v)
 #pragma unroll
-                for(int r = 0; r < 4; ++r)
-                    bq[v][r]
-                        = gload(p + int64_t(min(v0 + PNC * v + mfma_row<T>(q, r), nvec - 1)) * bv);
+                for(int r = 0; r < NR; ++r)
+                    bq[v][r] = gload(p + int64_t(min(v0 + PNC * v + group_vec(q, r), nvec - 1)) * bv);
         }
     }
 
@@ -358,11 +456,12 @@ struct PanelSolver
 #pragma unroll
         for(int v = 0; v < NVG; ++v)
         {
-            const T* p = Bb + int64_t(min(v0 + PNC * v + g, nvec - 1)) * bv
-                         + int64_t(PNC * ev + 4 * q) * br;
+            const T* p = Bb + int64_t(min(v0 + PNC * v + row_vec(g), nvec - 1)) * bv
+                         + int64_t(PNC * ev + 4 * q + kx) * br;
 #pragma unroll
             for(int kk = 0; kk < 4; ++kk)
-                y[v][kk] = gload(p + int64_t(kk) * br);
+                y[v][kk] = MODE == PM_CHAIN ? coherent_load(p + int64_t(kk) * bk)
+                                            : gload(p + int64_t(kk) * bk);
         }
     }
 
@@ -444,7 +543,7 @@ struct PanelSolver
 #pragma unroll
             for(int v = 0; v < NVG; ++v)
 #pragma unroll
-                for(int r = 0; r < 4; ++r)
+                for(int r = 0; r < NR; ++r)
                     c[v][r] = fma(__shfl(c[v][r] * dg, 16 * q + j, WAVE), l, c[v][r]);
         }
     }
@@ -461,17 +560,17 @@ struct PanelSolver
 #pragma unroll
         for(int v = 0; v < NVG; ++v)
 #pragma unroll
-            for(int r = 0; r < 4; ++r)
+            for(int r = 0; r < NR; ++r)
                 c[v][r] = fma(scale, bq[v][r], C[I][v][r]);
         if(scaled)
-            SolveSteps<T, NVG, 0>::run(c, Ld);
+            SolveSteps<T, NVG, NR, 0>::run(c, Ld);
         else
             solve_unscaled(c, t);
-        T* p = Y + (t % PRING) * YS + g;
+        T* p = Y + (t % PRING) * YS + (g ^ kx);
 #pragma unroll
         for(int v = 0; v < NVG; ++v)
 #pragma unroll
-            for(int r = 0; r < 4; ++r)
+            for(int r = 0; r < NR; ++r)
             {
                 c[v][r] *= dg;
                 p[v * YV + mfma_row<T>(q, r) * YP] = -c[v][r];
@@ -484,7 +583,7 @@ struct PanelSolver
         asm volatile("" : "+v"(qs));
         const int row = PNC * t + g;
         T*        b   = Bb + int64_t(row) * br;
-        if(WIDE && full_rows)
+        if(WIDE && NR == 4 && MODE != PM_CHAIN && full_rows)
         {
             if(row < K)
             {
@@ -497,11 +596,16 @@ struct PanelSolver
 #pragma unroll
         for(int v = 0; v < NVG; ++v)
 #pragma unroll
-            for(int r = 0; r < 4; ++r)
+            for(int r = 0; r < NR; ++r)
             {
-                const int vec = v0 + PNC * v + mfma_row<T>(qs, r);
+                const int vec = v0 + PNC * v + group_vec(qs, r);
                 if(row < K && vec < nvec)
-                    gstore(b + int64_t(vec) * bv, c[v][r]);
+                {
+                    if constexpr(MODE == PM_CHAIN)
+                        coherent_store(b + int64_t(vec) * bv, c[v][r]);
+                    else
+                        gstore(b + int64_t(vec) * bv, c[v][r]);
+                }
             }
     }
 
@@ -540,6 +644,8 @@ struct PanelSolver
                         ++e;
                     }
                 }
+                if constexpr(MODE == PM_CHAIN)
+                    raise(t);
             }
             segments<I + 1>(mine);
         }
@@ -585,7 +691,9 @@ struct PanelSolver
             }
         }
         e = 0;
-        if(MULTI && sb > 0)
+        if(MODE == PM_CHAIN && sb > 0)
+            early_chain(mine);
+        if(MODE == PM_MULTI && sb > 0)
         {
             // the earlier super-blocks' solution, without a chain
             T yf[NVG][4], yn[NVG][4];
@@ -602,6 +710,78 @@ struct PanelSolver
             }
         }
         segments<0>(mine);
+    }
+
+    // y_t is in B: this wavefront's stores are complete (they are write-through),
+    // then its flag says so
+    __device__ __forceinline__ void raise(int t)
+    {
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __hip_atomic_store(link + w, unsigned(t / 4 + 1), __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_AGENT);
+    }
+
+    // Sub-blocks 0..count - 1 are in B once flag i has passed those of wavefront i
+    __device__ __forceinline__ unsigned read_flags() const
+    {
+        return __hip_atomic_load(link + (g & 3), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    __device__ __forceinline__ int count_of(unsigned f) const
+    {
+        const int n  = int(4 * f) + (g & 3);
+        const int n0 = __builtin_amdgcn_readlane(n, 0), n1 = __builtin_amdgcn_readlane(n, 1);
+        const int n2 = __builtin_amdgcn_readlane(n, 2), n3 = __builtin_amdgcn_readlane(n, 3);
+        return min(min(n0, n1), min(n2, n3));
+    }
+    __device__ __forceinline__ void wait_avail(int ev)
+    {
+        const int need = ev + pw.bias;
+        for(int it = 0; avail <= need; ++it)
+        {
+            avail = count_of(read_flags());
+            if(it >= pw.spin_limit && avail <= need)
+            {
+                if(pw.err)
+                    __hip_atomic_store(pw.err, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+                avail = 0x7fffffff;
+            }
+        }
+        asm volatile("" ::: "memory"); // B is read after the flags
+    }
+
+    // The earlier super-blocks' solution as their workgroups publish it: y of
+    // the next sub-block is in flight during the products of one wherever it
+    // is known to be there, and the flags are read beside the products where
+    // it is not.
+    __device__ __forceinline__ void early_chain(int mine)
+    {
+        T    yf[NVG][4], yn[NVG][4];
+        bool have = false;
+        for(; e < sb; ++e)
+        {
+            if(!have)
+            {
+                wait_avail(e);
+                load_y(yn, e);
+            }
+#pragma unroll
+            for(int v = 0; v < NVG; ++v)
+#pragma unroll
+                for(int kk = 0; kk < 4; ++kk)
+                    yf[v][kk] = -yn[v][kk];
+            have = e + 1 < sb && avail > e + 1 + pw.bias;
+            if(have)
+            {
+                load_y(yn, e + 1);
+                early<0>(yf, mine);
+            }
+            else
+            {
+                const unsigned f = read_flags();
+                early<0>(yf, mine);
+                avail = max(avail, count_of(f));
+            }
+        }
     }
 
     // one sub-block of an earlier super-block, applied to every own tile
@@ -623,7 +803,7 @@ struct PanelSolver
 
     __device__ __forceinline__ void run(const T* Ap, T* Bp, int K_, int nvec_, int lda, int ldb,
                                         int flags, T scale_, int v0_, unsigned char* smem,
-                                        PanelWait pw_)
+                                        PanelWait pw_, unsigned* link_ = nullptr, int sb_ = 0)
     {
         const bool tA   = flags & SF_TA;
         const bool rev  = flags & SF_REV;
@@ -644,7 +824,9 @@ struct PanelSolver
         cs              = s * (tA ? 1 : lda);
         br              = s * (cols ? 1 : ldb);
         bv              = cols ? ldb : 1;
-        lq              = int64_t(4 * q) * cs;
+        kx              = KC && rev ? 3 : 0;
+        bk              = kx ? -br : br;
+        lq              = int64_t(4 * q + kx) * cs;
         Ab              = Ap + (rev ? int64_t(K - 1) * (int64_t(lda) + 1) : 0);
         Bb              = Bp + (rev ? int64_t(K - 1) * (cols ? 1 : ldb) : 0);
         Y               = reinterpret_cast<T*>(smem);
@@ -653,13 +835,23 @@ struct PanelSolver
         pw              = pw_;
         seen            = 0;
         if(threadIdx.x == 0)
-            *done = 0;
+            *done = sb_;
         __syncthreads();
-        sb = 0;
-        if constexpr(!MULTI)
+        if constexpr(MODE == PM_CHAIN)
+        {
+            link  = link_;
+            avail = 0;
+            sb    = sb_;
+            seen  = sb; // the counter starts where this super-block does
+            super_block((min(4 * NT, nsub - sb) - w + 3) / 4);
+        }
+        else if constexpr(MODE == PM_SINGLE)
+        {
+            sb = 0;
             super_block((nsub - w + 3) / 4);
+        }
         else
-            for(; sb < nsub; sb += 4 * NT)
+            for(sb = 0; sb < nsub; sb += 4 * NT)
             {
                 // the earlier super-blocks' stores to B are visible, the ring is free
                 if(sb > 0)
@@ -669,5 +861,23 @@ struct PanelSolver
         __syncthreads(); // LDS reuse by the caller's next panel
     }
 };
+
+// One panel, by the storage order of its triangle.
+template <typename T, int NT, int NVG, PanelMode MODE, int NR = 4, typename... Rest>
+__device__ __forceinline__ void panel_solve(const T* Ap, T* Bp, int K, int nvec, int lda, int ldb,
+                                            int flags, T scale, int v0, unsigned char* smem,
+                                            PanelWait pw, Rest... rest)
+{
+    if(flags & SF_TA)
+    {
+        PanelSolver<T, NT, NVG, MODE, NR, true> s;
+        s.run(Ap, Bp, K, nvec, lda, ldb, flags, scale, v0, smem, pw, rest...);
+    }
+    else
+    {
+        PanelSolver<T, NT, NVG, MODE, NR, false> s;
+        s.run(Ap, Bp, K, nvec, lda, ldb, flags, scale, v0, smem, pw, rest...);
+    }
+}
 } // namespace panel
 } // namespace rbamd

@@ -202,10 +202,8 @@ __global__ void __launch_bounds__(panel::PNT) __attribute__((amdgpu_waves_per_eu
             if(alpha == T(0))
                 panel::panel_zero<T>(Bp, k, nv, ldb, flags, p * panel::PNC, panel::PNC);
             else
-            {
-                panel::PanelSolver<T, 4, 1, true> s;
-                s.run(Ap, Bp, k, nv, lda, ldb, flags, alpha, p * panel::PNC, vb_smem, pw);
-            }
+                panel::panel_solve<T, 4, 1, panel::PM_MULTI>(
+                    Ap, Bp, k, nv, lda, ldb, flags, alpha, p * panel::PNC, vb_smem, pw);
         }
     }
 }
