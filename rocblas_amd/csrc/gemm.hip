@@ -1047,7 +1047,9 @@ static bool gemm_dma_eligible(const GemmArgsT<float, float, float>& a, int bk)
 // The DMA kernel's conditions: plain FP64 operands, 16-byte aligned rows; at
 // most one triangular operand, square (K x K), and then at most one of the
 // two operands transposed.
-static bool gemm_dma_eligible(const GemmArgsT<double, double, double>& a, int bk)
+// (tt: the balanced kernels, which take both transposed -- the uneven group of
+// trtri -- instead of A alone).
+static bool gemm_dma_eligible(const GemmArgsT<double, double, double>& a, int bk, bool tt = false)
 {
     auto al16 = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
     // an x-contiguous operand is loaded two rows of op() at a time
@@ -1057,7 +1059,7 @@ static bool gemm_dma_eligible(const GemmArgsT<double, double, double>& a, int bk
     const bool tri_ok  = !a.tri
                         || ((kind == GT_A_LOWER || kind == GT_A_UPPER || kind == GT_B_LOWER
                              || kind == GT_B_UPPER)
-                            && !(a.opA == 1 && a.opB == 1)
+                            && !(a.opA == 1 && a.opB == (tt ? 0 : 1))
                             && (!(a.tri & (GT_A_LOWER | GT_A_UPPER)) || a.M == a.K)
                             && (!(a.tri & (GT_B_LOWER | GT_B_UPPER)) || a.N == a.K));
     return tri_ok && a_pairs && b_pairs && a.K >= bk && a.K % bk == 0 && a.lda % 2 == 0
@@ -1333,7 +1335,7 @@ static int64_t balanced_shape_workgroups(rocblas_handle h, int M, int N, int K, 
 // split and the workspace holds its 2 W partial tiles.
 static int64_t balanced_workgroups(rocblas_handle h, const GemmArgsT<double, double, double>& a)
 {
-    if(!a.tri || !a.split_ok || !a.split_ws || !gemm_dma_eligible(a, 8))
+    if(!a.tri || !a.split_ok || !a.split_ws || !gemm_dma_eligible(a, 8, true))
         return 0;
     const int64_t W = balanced_shape_workgroups(h, a.M, a.N, a.K, a.tri, a.batch);
     return 2 * W <= a.split_ws_tiles ? W : 0;
@@ -1361,7 +1363,7 @@ static void launch_balanced_kind(rocblas_handle h, const GemmArgsT<double, doubl
     if(d.opA == 0 && d.opB == 0)
         launch_balanced_ops<0, 0, TRI>(h, d);
     else if(d.opA == 1)
-        launch_balanced_ops<1, 0, TRI>(h, d);
+        launch_balanced_ops<1, 1, TRI>(h, d);
     else
         launch_balanced_ops<0, 1, TRI>(h, d);
 }

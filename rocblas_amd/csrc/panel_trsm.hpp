@@ -259,7 +259,9 @@ enum PanelMode
 {
     PM_SINGLE, // it has at most 64 NT rows: one super-block
     PM_MULTI,  // this workgroup solves its super-blocks one after another
-    PM_CHAIN   // each super-block has a workgroup of its own (chain_trsm.hip)
+    PM_CHAIN,  // each super-block has a workgroup of its own (chain_trsm.hip)
+    PM_INVERSE // one super-block whose right-hand side is the unit vectors 0..15
+               // of canonical order (trtri_panel.hip): B is only written
 };
 
 // Flags of a panel of the chained solve, in device memory: word w counts the
@@ -433,6 +435,13 @@ struct PanelSolver
     // right-hand sides of sub-block t
     __device__ __forceinline__ void load_rhs(int t)
     {
+        if constexpr(MODE == PM_INVERSE)
+        {
+#pragma unroll
+            for(int r = 0; r < NR; ++r)
+                bq[0][r] = PNC * t + g == group_vec(q, r) ? T(1) : T(0);
+            return;
+        }
         const T* p = Bb + int64_t(min(PNC * t + g, K - 1)) * br;
         if(WIDE && NR == 4 && MODE != PM_CHAIN && full_rows)
         {
@@ -824,11 +833,15 @@ struct PanelSolver
         cs              = s * (tA ? 1 : lda);
         br              = s * (cols ? 1 : ldb);
         bv              = cols ? ldb : 1;
+        if constexpr(MODE == PM_INVERSE)
+            bv = s * ldb; // the columns of the inverse are reversed with its rows
         kx              = KC && rev ? 3 : 0;
         bk              = kx ? -br : br;
         lq              = int64_t(4 * q + kx) * cs;
         Ab              = Ap + (rev ? int64_t(K - 1) * (int64_t(lda) + 1) : 0);
         Bb              = Bp + (rev ? int64_t(K - 1) * (cols ? 1 : ldb) : 0);
+        if constexpr(MODE == PM_INVERSE)
+            Bb = Bp + (rev ? int64_t(K - 1) * (int64_t(ldb) + 1) : 0);
         Y               = reinterpret_cast<T*>(smem);
         D               = Y + PRING * YS + w * PNC * (YP + 1);
         done            = reinterpret_cast<int*>(Y + PRING * YS + 4 * PNC * (YP + 1));
@@ -845,7 +858,7 @@ struct PanelSolver
             seen  = sb; // the counter starts where this super-block does
             super_block((min(4 * NT, nsub - sb) - w + 3) / 4);
         }
-        else if constexpr(MODE == PM_SINGLE)
+        else if constexpr(MODE == PM_SINGLE || MODE == PM_INVERSE)
         {
             sb = 0;
             super_block((nsub - w + 3) / 4);

@@ -18,6 +18,15 @@
 
 namespace rbamd
 {
+// Order of the diagonal blocks inverted before the doubling: 16 and 32 by one
+// wavefront each, above by the panel solve, whose 512-row blocks take less
+// time than 256-row ones and a level of products (n = 3000 FP64: 610 us with
+// blocks of 32, of which the levels up to 256 rows took 125).
+static int trtri_block(int n)
+{
+    return n <= 16 ? 16 : n <= kTrtriNB ? kTrtriNB : n <= 256 ? 256 : kTrtriPanelNB;
+}
+
 // Workspace the balanced split products of an order-n inversion use: the
 // largest need of any FP64 doubling product (trtri_core's levels; equal
 // groups as the batch when `groups_batched`), 0 for FP32.
@@ -29,7 +38,7 @@ size_t trtri_split_bytes(rocblas_handle h, int n, int batch, bool groups_batched
     else
     {
         size_t need = 0;
-        for(int64_t s = (n <= 16 ? 16 : kTrtriNB); s < n; s *= 2)
+        for(int64_t s = trtri_block(n); s < n; s *= 2)
         {
             const int64_t full = n / (2 * s), n2last = n - full * 2 * s - s;
             if(full > 0)
@@ -248,8 +257,8 @@ rocblas_status trtri_double_step(rocblas_handle    h,
 }
 } // namespace
 
-// Blocked inversion in k^3/3 flops: the diagonal blocks of order kTrtriNB
-// are inverted by trtri_diag_kernel in one launch, then the inverse is built
+// Blocked inversion in k^3/3 flops: the diagonal blocks (trtri_block) are
+// inverted in one launch, then the inverse is built
 // bottom-up by doubling: at level s the groups of 2s rows (the last may be
 // shorter) get their off-diagonal block from two triangular-masked GEMMs
 // (trtri_double_step), all equal groups of a level in one batched launch
@@ -291,11 +300,12 @@ rocblas_status trtri_core(rocblas_handle    handle,
     d.X     = invA;
     d.ldx   = ldinvA;
     d.n     = n;
-    d.nb    = n <= 16 ? 16 : kTrtriNB;
+    d.nb    = trtri_block(n);
     d.upper = upper;
     d.unit  = diag == rocblas_diagonal_unit;
     d.batch = batch_count;
-    rocblas_status st = trtri_diag_launch<T>(handle, d);
+    rocblas_status st = n <= kTrtriNB ? trtri_diag_launch<T>(handle, d)
+                                      : trtri_panel_launch<T>(handle, d);
     if(st != rocblas_status_success || n <= d.nb)
         return st;
 

@@ -6,10 +6,12 @@
 
 namespace rbamd
 {
-// Order of the diagonal blocks the inversion kernel handles for n > 16 (its
-// FP64 form holds a 32-entry column per lane without spilling; larger
-// blocks are left to the doubling steps, whose GEMMs carry the flops).
+// Largest order the one-wavefront inversion kernel handles (its FP64 form holds
+// a 32-entry column per lane without spilling).
 constexpr int kTrtriNB = 32;
+
+// Largest diagonal blocks the panel solve inverts (trtri_panel.hip).
+constexpr int kTrtriPanelNB = 512;
 
 // Diagonal blocks [b nb, min(n, (b+1) nb)) of n x n triangles: A (lda) and
 // the inverse X (ldx), batch instances.
@@ -21,7 +23,7 @@ struct TrtriDiagArgs
     BatchPtr<T>       X;
     int               ldx;
     int               n;
-    int               nb; // 1..kTrtriNB
+    int               nb; // block order
     int               upper;
     int               unit;
     int               batch;
@@ -31,6 +33,10 @@ struct TrtriDiagArgs
 // block := 0); X is only written.
 template <typename T>
 rocblas_status trtri_diag_launch(rocblas_handle h, const TrtriDiagArgs<T>& a);
+
+// The same for blocks of up to kTrtriPanelNB rows, by the panel solve.
+template <typename T>
+rocblas_status trtri_panel_launch(rocblas_handle h, const TrtriDiagArgs<T>& a);
 
 // X's strictly-opposite triangle outside the diagonal blocks := 0 (A unused).
 template <typename T>
