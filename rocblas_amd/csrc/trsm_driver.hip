@@ -183,7 +183,7 @@ constexpr int SMALL_K = 64; // granularity of the recursion's splits
 
 // leaves of the recursion for right-hand sides of at least kWidePanels panels
 constexpr int kWideLeafK  = 256;
-constexpr int kWidePanels = 64;
+constexpr int kWidePanels = 512;
 
 template <typename T>
 struct Solver
@@ -289,10 +289,12 @@ struct Solver
         const int K = b - a;
         if(K <= kSmallMaxK)
             return leaf(a, b);
-        // A panel leaf streams its whole triangle once per 16-vector panel;
-        // with many panels the work is better spent in GEMM updates, so wide
-        // right-hand sides stop at leaves of kWideLeafK rows (measured at
-        // m = n = 1024..16384: 186 vs 202 us at 1024^2, 506 vs 544 us at 2048^2).
+        // A panel leaf streams its whole triangle once per 16 or 32 vectors and
+        // leaves the matrix cores idle along its chain; with many panels the
+        // work is better spent in GEMM updates, so wide right-hand sides stop at
+        // leaves of kWideLeafK rows.  Measured with leaves of 256 / 512 rows:
+        // 2048^2 276 / 263 us, FP32 3001 x 2999 626 / 536 us, 16384^2 67.5 / 67.8
+        // ms (leaves of 128: 329 us, 787 us, 68.1 ms).
         const int64_t panels = int64_t((sideL ? p.n : p.m) + 15) / 16 * p.batch;
         if(panel_fits<T>(h, K) && (K <= kWideLeafK || panels < kWidePanels))
             return panel_leaf(a, b);
