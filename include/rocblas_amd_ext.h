@@ -31,8 +31,7 @@ typedef enum rocblas_amd_synth_dist_
  * with its own m[i], n[i], lda[i], ldb[i].  m, n, lda, ldb, A and B are device
  * arrays of batch_count entries; alpha is one scalar (host or device per the
  * pointer mode).  A one-workgroup planning launch orders the work by cost and
- * two persistent launches solve it (k <= 512 with the MFMA panel solve, larger
- * triangles one wavefront each); the call allocates nothing beyond the handle
+ * one persistent launch solves it with the MFMA panel solve; the call allocates nothing beyond the handle
  * workspace (36 bytes per instance + 64; batch_count < 2^28) and can be
  * captured in a HIP graph.  No counterpart in the reference: rocBLAS callers
  * loop over rocblas_dtrsm.  The per-instance sizes are device data, so they

@@ -1,5 +1,6 @@
 // panel_trsm.hpp -- the panel solve shared by the single-launch k <= 512
-// path (panel_trsm.hip) and the persistent variable-size batch (vbatched.hip).
+// path (panel_trsm.hip), the persistent variable-size batch (vbatched.hip), the
+// chained solve (chain_trsm.hip) and the inverses of trtri (trtri_panel.hip).
 //
 // PanelSolver<T, NT, NVG> solves 16 * NVG right-hand-side vectors of one
 // instance with all four wavefronts of a workgroup.  Canonical form as in
@@ -49,7 +50,11 @@ namespace panel
 {
 constexpr int PNC   = 16;  // vectors per vector group, rows per sub-block
 constexpr int PNT   = 256; // threads
-constexpr int PRING = 8;   // LDS slots of solved sub-blocks
+// LDS slots of solved sub-blocks.  The owner of t writes its slot after it has
+// read y_{t-1}; each publisher in that chain had finished reading everything up
+// to two sub-blocks before its own, and every other wavefront with sub-blocks
+// left published one of the last three, so none still reads t - 5 or earlier.
+constexpr int PRING = 8;
 
 // Row pitch (elements) of a solved sub-block in LDS, [vector][row]: a lane
 // reads four consecutive rows of a vector as 16-byte words, conflict-free.
