@@ -10,8 +10,8 @@
 // over rocblas_dtrsm (one to thirty launches per instance).
 //
 // Plan kernel (1 workgroup): every valid instance becomes up to
-// kVbPanelGroups work items, each a strided share of the instance's 16-vector
-// panels; the items are counting-sorted by cost bucket
+// kVbPanelGroups work items, each a strided share of the instance's pieces of 16
+// or 32 vectors; the items are counting-sorted by cost bucket
 // (floor(log2(k^2 * vectors))), largest first.  The work counter is reset
 // with a plain store (no memset node in a graph).
 //
@@ -52,6 +52,7 @@ struct VbArgs
     const T*           alpha_arr;
     int*               items;   // workspace: panel work items (inst * 8 + group, groups * batch)
     int*               counter; // workspace: [0] items taken, [1] items
+    int                unit;    // vectors solved at a time: 16 or 32
     int                groups[kVbPanelBuckets]; // work items per instance of the panel
                                                 // kernel (1..8), by size bucket of k
 };
@@ -112,8 +113,8 @@ __device__ __forceinline__ bool vb_shape(const VbArgs<T>& a, int i, int& k, int&
 template <typename T>
 __device__ __forceinline__ int vb_groups(const VbArgs<T>& a, int k, int nv)
 {
-    const int panels = (nv + panel::PNC - 1) / panel::PNC;
-    return min(panels, a.groups[vb_panel_bucket(k)]);
+    const int units = (nv + a.unit - 1) / a.unit;
+    return min(units, a.groups[vb_panel_bucket(k)]);
 }
 
 template <typename T>
@@ -130,8 +131,8 @@ __global__ void __launch_bounds__(1024) vb_plan_kernel(const VbArgs<T> a)
         if(!vb_shape(a, i, k, nv))
             continue;
         const int G   = vb_groups(a, k, nv);
-        const int per = ((nv + panel::PNC - 1) / panel::PNC + G - 1) / G;
-        atomicAdd(&hist[vb_cost_bucket(k, min(nv, per * panel::PNC))], G);
+        const int per = ((nv + a.unit - 1) / a.unit + G - 1) / G;
+        atomicAdd(&hist[vb_cost_bucket(k, min(nv, per * a.unit))], G);
     }
     __syncthreads();
     if(threadIdx.x == 0)
@@ -152,8 +153,8 @@ __global__ void __launch_bounds__(1024) vb_plan_kernel(const VbArgs<T> a)
         if(!vb_shape(a, i, k, nv))
             continue;
         const int G   = vb_groups(a, k, nv);
-        const int per = ((nv + panel::PNC - 1) / panel::PNC + G - 1) / G;
-        const int pos = atomicAdd(&offs[vb_cost_bucket(k, min(nv, per * panel::PNC))], G);
+        const int per = ((nv + a.unit - 1) / a.unit + G - 1) / G;
+        const int pos = atomicAdd(&offs[vb_cost_bucket(k, min(nv, per * a.unit))], G);
         for(int g = 0; g < G; ++g)
             a.items[pos + g] = i * 8 + g;
     }
@@ -164,7 +165,7 @@ template <typename T>
 __global__ void __launch_bounds__(panel::PNT) __attribute__((amdgpu_waves_per_eu(2)))
     vb_panel_kernel(const VbArgs<T> a, panel::PanelWait pw)
 {
-    __shared__ __align__(16) unsigned char vb_smem[panel::lds_bytes<T, 1>()];
+    __shared__ __align__(16) unsigned char vb_smem[panel::lds_bytes<T, 2>()];
     __shared__ int item_s;
     const int      total = a.counter[1];
     if(int(blockIdx.x) >= total)
@@ -189,7 +190,7 @@ __global__ void __launch_bounds__(panel::PNT) __attribute__((amdgpu_waves_per_eu
         k  = __builtin_amdgcn_readfirstlane(k);
         nv = __builtin_amdgcn_readfirstlane(nv);
         const int G      = vb_groups(a, k, nv);
-        const int panels = (nv + panel::PNC - 1) / panel::PNC;
+        const int units  = (nv + a.unit - 1) / a.unit;
         // per-instance values read from device arrays are uniform too
         const T*  Ap     = uniform_ptr(a.A[inst]);
         T*        Bp     = uniform_ptr(a.B[inst]);
@@ -197,21 +198,36 @@ __global__ void __launch_bounds__(panel::PNT) __attribute__((amdgpu_waves_per_eu
         const int flags  = uniform_int(vb_flags(a, inst));
         const int lda    = uniform_int(a.lda[inst]);
         const int ldb    = uniform_int(a.ldb[inst]);
-        for(int p = g; p < panels; p += G)
+        for(int p = g; p < units; p += G)
         {
+            const int v0 = p * a.unit;
             if(alpha == T(0))
-                panel::panel_zero<T>(Bp, k, nv, ldb, flags, p * panel::PNC, panel::PNC);
+                panel::panel_zero<T>(Bp, k, nv, ldb, flags, v0, a.unit);
+            else if(a.unit > panel::PNC && nv - v0 > panel::PNC)
+                panel::panel_solve<T, 4, 2, panel::PM_MULTI>(Ap, Bp, k, nv, lda, ldb, flags, alpha,
+                                                             v0, vb_smem, pw);
             else
-                panel::panel_solve<T, 4, 1, panel::PM_MULTI>(
-                    Ap, Bp, k, nv, lda, ldb, flags, alpha, p * panel::PNC, vb_smem, pw);
+                panel::panel_solve<T, 4, 1, panel::PM_MULTI>(Ap, Bp, k, nv, lda, ldb, flags, alpha,
+                                                             v0, vb_smem, pw);
         }
     }
 }
+
+// 32 vectors at a time read a triangle half as often and leave half as many,
+// longer items, so the chip must stay full of them: from 8 instances per CU on.
+// The results are the same bits.  Measured on 256 CUs, 16 / 32 vectors at a
+// time, us, k log-uniform in [8, 512], FP64 up to 64 vectors, FP32 the same, FP64
+// up to 20 vectors (the worst: 17 to 20 vectors take one item for two):
+// 300 instances 62 / 73, 51 / 59, 54 / 71; 1024 99 / 106, 77 / 73, 75 / 85;
+// 1500 150 / 132, 101 / 87, 95 / 102; 2048 210 / 175, 130 / 113, 122 / 123;
+// 4096 382 / 316, 266 / 221, 221 / 212.
+constexpr int kVbWideInstancesPerCu = 8;
 
 template <typename T>
 rocblas_status vbatched_launch(rocblas_handle h, VbArgs<T> a)
 {
     DeviceGuard g(h->device);
+    a.unit = a.batch / kVbWideInstancesPerCu >= h->num_cus ? 2 * panel::PNC : panel::PNC;
     hipLaunchKernelGGL(vb_plan_kernel<T>, dim3(1), dim3(1024), 0, h->stream, a);
     rocblas_status st = launch_status();
     if(st != rocblas_status_success)

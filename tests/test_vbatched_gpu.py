@@ -143,6 +143,31 @@ def test_random_against_oracle(h, side, uplo, trans):
         assert eta <= 1e-14, (i, m, n, eta)
 
 
+@pytest.mark.parametrize("prec", ["d", "s"])
+@pytest.mark.parametrize("side,uplo,trans", [("L", "L", "N"), ("L", "U", "T"), ("R", "L", "N")])
+def test_large_batch_bitwise(h, side, uplo, trans, prec):
+    """From 8 instances per CU on, an instance's vectors are solved 32 at a time:
+    the integer problem's X bit for bit, at vector counts around 16, 32 and 64
+    and triangles around the 64- and 256-row tiles, and the rest of the batch
+    (single rows) as well."""
+    rng = np.random.default_rng(4100 + ALL_CASES.index((side, uplo, trans)))
+    kv = [(k, v) for k in (5, 64, 65, 257) for v in (1, 16, 17, 32, 33, 48, 49, 64, 65)]
+    batch = 8 * torch.cuda.get_device_properties(0).multi_processor_count
+    kv += [(1, 17)] * (batch - len(kv))
+    shape = [(k, v) if side == "L" else (v, k) for k, v in kv]
+    say("vbatched large batch", side, uplo, trans, prec, batch)
+    probs = [integer_kat(side, uplo, trans, "U" if prec == "s" else "N", m, n, rng, lda=k + 1,
+                         ldb=m + 1) for (k, _), (m, n) in zip(kv, shape)]
+    P = VbProblem(side, [m for m, _ in shape], [n for _, n in shape], [p[0] for p in probs],
+                  [p[1] for p in probs], torch.float32 if prec == "s" else torch.float64)
+    assert P.run(h, side, uplo, trans, "U" if prec == "s" else "N", 1.0, prec) == S.success
+    torch.cuda.synchronize()
+    for i, (m, n) in enumerate(shape):
+        got = P.result(i)
+        assert np.array_equal(got[:m, :n], probs[i][2][:m, :n]), (i, m, n)
+        assert np.all(got[m:, :] == 0.0)
+
+
 @pytest.mark.parametrize("side,uplo,trans", [("L", "L", "N"), ("R", "U", "T")])
 def test_large_triangles_against_oracle(h, side, uplo, trans):
     """Triangles beyond 512 (up to 1100) in the same batch as small ones take
