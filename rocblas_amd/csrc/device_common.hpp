@@ -188,7 +188,8 @@ enum SmallFlags : int
     SF_UNIT  = 8,  // unit diagonal: the diagonal of A is never read
     SF_COLS  = 16, // the vectors are columns of B (side left)
     SF_SCALE = 32, // multiply the right-hand side by alpha
-    SF_FULL  = 64  // small-solve launch with K == KMAX and every slot holding 16 vectors
+    SF_FULL  = 64, // small-solve launch with K == KMAX and every slot holding 16 vectors
+    SF_TRANSPOSED = 128 // inverses only: written below the diagonal only, transposed
 };
 
 template <typename T>

@@ -297,6 +297,7 @@ struct PanelSolver
     int      K, nsub, nvec, v0;
     bool     unit;
     bool     full_rows; // the vectors are rows of B and all 16 NVG of them exist
+    bool     turned;    // PM_INVERSE: the result goes below the diagonal only, transposed
     T        scale;
     // wavefront and lane
     int     w, g, q;
@@ -613,7 +614,7 @@ struct PanelSolver
             for(int r = 0; r < NR; ++r)
             {
                 const int vec = v0 + PNC * v + group_vec(qs, r);
-                if(row < K && vec < nvec)
+                if(row < K && vec < nvec && (MODE != PM_INVERSE || !turned || row > vec))
                 {
                     if constexpr(MODE == PM_CHAIN)
                         coherent_store(b + int64_t(vec) * bv, c[v][r]);
@@ -838,15 +839,18 @@ struct PanelSolver
         cs              = s * (tA ? 1 : lda);
         br              = s * (cols ? 1 : ldb);
         bv              = cols ? ldb : 1;
-        if constexpr(MODE == PM_INVERSE)
-            bv = s * ldb; // the columns of the inverse are reversed with its rows
         kx              = KC && rev ? 3 : 0;
         bk              = kx ? -br : br;
         lq              = int64_t(4 * q + kx) * cs;
         Ab              = Ap + (rev ? int64_t(K - 1) * (int64_t(lda) + 1) : 0);
         Bb              = Bp + (rev ? int64_t(K - 1) * (cols ? 1 : ldb) : 0);
         if constexpr(MODE == PM_INVERSE)
-            Bb = Bp + (rev ? int64_t(K - 1) * (int64_t(ldb) + 1) : 0);
+        {
+            Bb     = Bp + (rev ? int64_t(K - 1) * (int64_t(ldb) + 1) : 0);
+            turned = flags & SF_TRANSPOSED;
+            bv     = s * (turned ? 1 : ldb); // the columns of the inverse are reversed with its rows
+            br     = s * (turned ? ldb : 1);
+        }
         Y               = reinterpret_cast<T*>(smem);
         D               = Y + PRING * YS + w * PNC * (YP + 1);
         done            = reinterpret_cast<int*>(Y + PRING * YS + 4 * PNC * (YP + 1));

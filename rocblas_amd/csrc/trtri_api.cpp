@@ -7,7 +7,8 @@
 // with triangular-masked MFMA GEMMs.  The triangle opposite `uplo` of invA
 // comes out exactly zero ("may be cleared", rocblas-functions.h:19064-19071).
 // When invA is A itself (in-place call), A is first copied to the handle
-// workspace.
+// workspace; pointer arrays that differ but hold the same matrices are found
+// on the device (trtri_panel.hip).
 #include "internal.hpp"
 #include "trtri_kernels.hpp"
 #include "device_common.hpp"

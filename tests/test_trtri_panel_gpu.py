@@ -68,3 +68,46 @@ def test_inverse_kernels_have_their_wait_states(tmp_path):
     found = {name: scan(body) for name, body in kernels(asm, "trtri_panel_kernel")}
     assert len(found) == 4, sorted(found)
     assert not any(found.values()), {k[:60]: v[:2] for k, v in found.items() if v}
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("prec", ["d", "s"])
+@pytest.mark.parametrize("uplo", ["L", "U"])
+def test_two_pointer_arrays_of_the_same_matrices(uplo, prec):
+    """In place through pointer arrays that differ: the host cannot see that some of their entries
+    are equal.  Such an instance gives the bits of the same call out of place."""
+    import torch
+    from tests.gpu_util import GpuHandle
+    h = GpuHandle()
+    rng = np.random.default_rng(17)
+    dt = np.float64 if prec == "d" else np.float32
+    for n, batch in ((33, 7), (48, 3), (200, 5), (256, 2), (300, 3), (512, 2), (600, 3), (200, 300)):
+        print("trtri in place, two arrays", prec, uplo, n, batch, flush=True)
+        ld = n + 3
+        A = oracle.diag_dominant_triangular(n, uplo, rng, lda=ld).astype(dt)
+        dA = torch.from_numpy(np.tile(np.nan_to_num(A).ravel(order="F"), batch)).cuda()
+        size = dA.element_size() * ld * n
+
+        def call(a, x):
+            pa = torch.tensor([a.data_ptr() + size * i for i in range(batch)]).cuda()
+            # every third instance of an in-place call goes to a matrix of its own
+            px = torch.tensor([(spare if i % 3 == 2 else x).data_ptr() + size * i
+                               for i in range(batch)]).cuda()
+            st = rb.trtri_batched(h, uplo, "N", n, pa.data_ptr(), ld, px.data_ptr(), ld, batch,
+                                  precision=prec)
+            assert st == rb.rocblas_status.success
+            return [t.cpu().numpy().reshape(batch, n, ld)[:, :, :n] for t in (x, spare)]
+
+        spare = torch.zeros_like(dA)
+        want, wspare = call(dA, torch.zeros_like(dA))
+        spare = torch.zeros_like(dA)
+        got, gspare = call(dA, dA)
+        for i in range(batch):
+            w, g = (wspare[i], gspare[i]) if i % 3 == 2 else (want[i], got[i])
+            assert np.array_equal(w, g), (n, i)
+        tri = np.asfortranarray(np.nan_to_num(A[:n]).astype(np.float64))
+        oracle.trtri(uplo, "N", n, tri)
+        tri = np.tril(tri) if uplo == "L" else np.triu(tri)
+        # clients/include/unit.hpp:631-638: eps * max(10000, n), relative
+        assert np.abs(got[0].T - tri).max() / np.abs(tri).max() <= np.finfo(dt).eps * max(10000, n)
+    h.close()
