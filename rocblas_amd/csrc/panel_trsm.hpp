@@ -187,6 +187,16 @@ __device__ __forceinline__ bool scaled_ok(float l, float s)
     return (__builtin_fabsf(s) <= 0x1p+120f) & ((__builtin_fabsf(s) >= 0x1p-120f) | (l == 0.0f));
 }
 
+// an infinity or NaN
+__device__ __forceinline__ bool not_finite(double x)
+{
+    return __builtin_amdgcn_class(x, 0x207);
+}
+__device__ __forceinline__ bool not_finite(float x)
+{
+    return __builtin_amdgcn_classf(x, 0x207);
+}
+
 // Bounds of the LDS waits.  Every wait ends by itself (all wavefronts of a
 // workgroup are resident, and the owner of the first unpublished sub-block
 // waits for published ones only); the poll limit turns a mistake into a
@@ -441,6 +451,10 @@ struct PanelSolver
     // right-hand sides of sub-block t
     __device__ __forceinline__ void load_rhs(int t)
     {
+        load_rhs(t, br, bv);
+    }
+    __device__ __forceinline__ void load_rhs(int t, int br, int bv)
+    {
         if constexpr(MODE == PM_INVERSE)
         {
 #pragma unroll
@@ -545,8 +559,11 @@ struct PanelSolver
         }
     }
 
-    // The unscaled substitution, for blocks prep_diag() refuses: x_J = c_J / L_JJ
-    // first, then c_i -= L_iJ x_J, column by column from memory.
+    // The unscaled substitution: x_J = c_J / L_JJ first, then c_i -= L_iJ x_J for
+    // the rows below only, column by column from memory.  For blocks that
+    // prep_diag() refuses, and for what is not finite after the scaled steps:
+    // those multiply the rows from J up by 0, which an infinity turns into NaN
+    // there too.
     __device__ __forceinline__ void solve_unscaled(T (&c)[NVG][4], int t)
     {
         const int below = PNC * t + g < K ? g : 0;
@@ -554,13 +571,42 @@ struct PanelSolver
         for(int j = 0; j < PNC - 1 && PNC * t + j < K; ++j)
         {
             const T x = gload(p + int64_t(j) * cs);
-            const T l = j < below ? -x : T(0);
 #pragma unroll
             for(int v = 0; v < NVG; ++v)
 #pragma unroll
                 for(int r = 0; r < NR; ++r)
-                    c[v][r] = fma(__shfl(c[v][r] * dg, 16 * q + j, WAVE), l, c[v][r]);
+                {
+                    const T    y   = __shfl(c[v][r] * dg, 16 * q + j, WAVE);
+                    const bool use = j < below && !above_unit(t, j, r);
+                    c[v][r]        = use ? fma(y, -x, c[v][r]) : c[v][r];
+                }
         }
+    }
+
+    // PM_INVERSE: row j of sub-block t is above the 1 of the unit vector in
+    // register r, so the inverse has a zero there (a zero pivot makes 0 / 0 of it)
+    __device__ __forceinline__ bool above_unit(int t, int j, int r) const
+    {
+        return MODE == PM_INVERSE && t == 0 && j < group_vec(q, r);
+    }
+
+    // y_t from the eliminated right-hand sides, and into its LDS slot (negated)
+    __device__ __forceinline__ void scale_y(T (&c)[NVG][4], int t) const
+    {
+#pragma unroll
+        for(int v = 0; v < NVG; ++v)
+#pragma unroll
+            for(int r = 0; r < NR; ++r)
+                c[v][r] = above_unit(t, g, r) ? T(0) : c[v][r] * dg;
+    }
+    __device__ __forceinline__ void write_y(const T (&c)[NVG][4], int t) const
+    {
+        T* p = Y + (t % PRING) * YS + (g ^ kx);
+#pragma unroll
+        for(int v = 0; v < NVG; ++v)
+#pragma unroll
+            for(int r = 0; r < NR; ++r)
+                p[v * YV + mfma_row<T>(q, r) * YP] = -c[v][r];
     }
 
     // own sub-block t (tile I) is final: solve, publish, store
@@ -579,19 +625,44 @@ struct PanelSolver
                 c[v][r] = fma(scale, bq[v][r], C[I][v][r]);
         if(scaled)
             SolveSteps<T, NVG, NR, 0>::run(c, Ld);
-        else
-            solve_unscaled(c, t);
-        T* p = Y + (t % PRING) * YS + (g ^ kx);
+        // A value that is not finite when its step reads it leaves none of its
+        // vector finite.  The checks run beside the LDS writes, where they cost
+        // up to 1% of a solve (512 x 256 35.4 -> 35.5 us; in front of the writes
+        // 36.5).
+        scale_y(c, t);
+        write_y(c, t);
+        uint64_t again = scaled ? 0 : 1;
 #pragma unroll
         for(int v = 0; v < NVG; ++v)
 #pragma unroll
             for(int r = 0; r < NR; ++r)
-            {
-                c[v][r] *= dg;
-                p[v * YV + mfma_row<T>(q, r) * YP] = -c[v][r];
-            }
+                again |= __builtin_amdgcn_ballot_w64(not_finite(c[v][r]));
         // the slot is written before the counter says so
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        if(__builtin_expect(again != 0, 0))
+        {
+            T d[NVG][4];
+            // (the right-hand sides are not kept during the steps; opaque
+            // strides, or their wider forms would be kept for the stores too)
+            int br_ = br, bv_ = bv;
+            asm volatile("" : "+s"(br_), "+s"(bv_));
+            load_rhs(t, br_, bv_);
+#pragma unroll
+            for(int v = 0; v < NVG; ++v)
+#pragma unroll
+                for(int r = 0; r < NR; ++r)
+                    d[v][r] = fma(scale, bq[v][r], C[I][v][r]);
+            solve_unscaled(d, t);
+            scale_y(d, t);
+            // finite results keep their bits whatever their neighbours hold
+#pragma unroll
+            for(int v = 0; v < NVG; ++v)
+#pragma unroll
+                for(int r = 0; r < NR; ++r)
+                    c[v][r] = scaled && !not_finite(c[v][r]) ? c[v][r] : d[v][r];
+            write_y(c, t);
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        }
         __hip_atomic_store(done, t + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
         // (opaque, so the addresses are not kept in registers all along)
         int qs = q;
