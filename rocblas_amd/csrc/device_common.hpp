@@ -203,6 +203,7 @@ struct SmallArgs
     int               ldb;
     int               chunks;    // ceil(nvec / vectors per slot)
     int64_t           units;     // batch * chunks
+    int64_t           unit0;     // first unit of the launch
     int               flags;
     int               bs_stride; // elements per staged vector (side L)
     T                 alpha_host;
@@ -214,7 +215,8 @@ constexpr int DPP_G  = 4;  // slots per wavefront
 
 // Single-launch panel solve for k <= kPanelMaxK (panel_trsm.hip): one workgroup
 // per 16 or 32 vectors, same SmallArgs (K, nvec, lda, ldb, flags, alpha);
-// `units` is ignored (the batch count is passed separately).
+// `units` and `unit0` are set by the launch (the batch count is passed
+// separately).
 constexpr int kPanelMaxK = 512;
 
 template <typename T>

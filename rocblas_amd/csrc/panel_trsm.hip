@@ -1,7 +1,8 @@
-// panel_trsm.hip -- single-launch solve for 64 < k <= 512 (and below 64 where
-// the driver prefers it): one workgroup per 16 or 32 right-hand-side vectors
-// of one instance (panel_trsm.hpp).  Workgroups are independent, so a whole
-// k <= 512 solve is one launch with no inter-workgroup communication.
+// panel_trsm.hip -- single-launch solve for 32 < k <= 512: one workgroup per 16
+// or 32 right-hand-side vectors of one instance (panel_trsm.hpp).  Workgroups
+// are independent, so a whole k <= 512 solve is one launch (2^23 workgroups at
+// a time) with no inter-workgroup communication.
+#include "launch_slices.hpp"
 #include "panel_trsm.hpp"
 
 namespace rbamd
@@ -19,7 +20,7 @@ __device__ __forceinline__ void panel_unit(const SmallArgs<T>& a, panel::PanelWa
     const T        scale = (a.flags & SF_SCALE) ? alpha : T(1);
     const unsigned qn = gridDim.x / 8, rn = gridDim.x % 8;
     const unsigned x = blockIdx.x % 8, l = blockIdx.x / 8;
-    const int64_t  unit = a.units + (x * qn + min(x, rn) + l);
+    const int64_t  unit = a.unit0 + (x * qn + min(x, rn) + l);
     const int64_t  b    = unit / a.chunks;
     const int      v0   = int(unit - b * a.chunks) * panel::PNC * NVG;
     T*             Bp   = a.B.get(b);
@@ -83,10 +84,10 @@ rocblas_status launch_panel(rocblas_handle h, const SmallArgs<T>& a, int batch)
     s.chunks       = (a.nvec + panel::PNC * nvg - 1) / (panel::PNC * nvg);
     const int64_t          units = int64_t(batch) * s.chunks;
     const panel::PanelWait pw    = panel::panel_wait(h);
-    // `units` of the kernel argument is the launch's first work unit
-    for(s.units = 0; s.units < units; s.units += 1 << 30)
-    {
-        const dim3 grid(unsigned(std::min<int64_t>(units - s.units, 1 << 30)));
+    s.units                      = units;
+    for_launch_slices(units, panel::PNT, [&](int64_t first, unsigned count) {
+        const dim3 grid(count);
+        s.unit0 = first;
         if(a.K > 256 && nvg == 1)
             hipLaunchKernelGGL(panel_trsm_kernel<T>, grid, dim3(panel::PNT), 0, h->stream, s, pw);
         else if(a.K > 256)
@@ -97,7 +98,7 @@ rocblas_status launch_panel(rocblas_handle h, const SmallArgs<T>& a, int batch)
         else
             hipLaunchKernelGGL((panel_short_kernel<T, 2>), grid, dim3(panel::PNT), 0, h->stream, s,
                                pw);
-    }
+    });
     return launch_status();
 }
 

@@ -84,7 +84,7 @@ __host__ __device__ constexpr int lofs(int i, int j)
 // with more than 16 vectors occupies several slots, each loading the
 // triangle (the duplicate loads are the same addresses in one instruction).
 //
-// Slot bookkeeping is wave-uniform: slot s is unit blockIdx.x * 4 + s, and
+// Slot bookkeeping is wave-uniform: slot s is unit unit0 + blockIdx.x * 4 + s, and
 // its instance pointers and first vector are read into scalar registers.
 // Side L loads B coalesced down the columns -- load step s covers
 // 64 / KMAX whole columns of one slot -- so every address is a per-lane
@@ -166,7 +166,7 @@ __global__ void __launch_bounds__(WAVE) small_trsm_dpp_kernel(const SmallArgs<T>
 
     if(lane < G)
     {
-        const int64_t u = int64_t(blockIdx.x) * G + lane;
+        const int64_t u = a.unit0 + int64_t(blockIdx.x) * G + lane;
         if(u < a.units)
         {
             const int64_t inst = a.chunks == 1 ? u : u / a.chunks;

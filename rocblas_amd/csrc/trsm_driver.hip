@@ -17,6 +17,7 @@
 // synchronisation, graph-capturable); alpha == 0 writes B := 0 and leaves A
 // unread (library/include/internal/rocblas-functions.h:19357-19361).
 #include "device_common.hpp"
+#include "launch_slices.hpp"
 
 namespace rbamd
 {
@@ -161,19 +162,16 @@ static rocblas_status launch_small(rocblas_handle h, const SmallArgs<T>& args_in
     const size_t lds     = cols ? size_t(WAVE) * a.bs_stride * sizeof(T) : 0; // staging
     if(a.K == kmax && a.nvec % DPP_VP == 0 && a.units % DPP_G == 0)
         a.flags |= SF_FULL;
-    const int64_t blocks = (a.units + DPP_G - 1) / DPP_G;
-    if(blocks > int64_t(0x7fffffff))
-        return rocblas_status_invalid_size;
-    const dim3 grid{unsigned(blocks)};
-    switch(kmax)
-    {
-    case 8:
-        return launch_small_kmax<T, 8>(h, a, grid, lds);
-    case 16:
-        return launch_small_kmax<T, 16>(h, a, grid, lds);
-    default:
-        return launch_small_kmax<T, 32>(h, a, grid, lds);
-    }
+    const int64_t  blocks = (a.units + DPP_G - 1) / DPP_G;
+    rocblas_status st     = rocblas_status_success;
+    for_launch_slices(blocks, WAVE, [&](int64_t first, unsigned count) {
+        a.unit0 = first * DPP_G;
+        if(st == rocblas_status_success)
+            st = kmax == 8    ? launch_small_kmax<T, 8>(h, a, dim3(count), lds)
+                 : kmax == 16 ? launch_small_kmax<T, 16>(h, a, dim3(count), lds)
+                              : launch_small_kmax<T, 32>(h, a, dim3(count), lds);
+    });
+    return st;
 }
 
 // ---------------------------------------------------------------------------

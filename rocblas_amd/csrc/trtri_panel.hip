@@ -21,6 +21,7 @@
 // 32 joined by doubling products of 32 to 256 rows, two launches per level.
 // Measured on MI355X, FP64, us: n = 64 22 -> 4.8, 256 48 -> 13.5, 512 72 -> 34,
 // 1024 121 -> 83; 500 instances of order 200 303 -> 95.
+#include "launch_slices.hpp"
 #include "panel_trsm.hpp"
 #include "trtri_kernels.hpp"
 
@@ -131,23 +132,22 @@ rocblas_status trtri_panel_launch(rocblas_handle h, const TrtriDiagArgs<T>& a)
     const int     panels = (std::min(a.n, a.nb) + panel::PNC - 1) / panel::PNC;
     const int64_t units  = int64_t(a.batch) * nblk * panels;
     const auto    pw     = panel::panel_wait(h);
-    for(int64_t u = 0; u < units; u += 1 << 30)
-    {
-        const dim3 grid(unsigned(std::min<int64_t>(units - u, 1 << 30)));
+    for_launch_slices(units, panel::PNT, [&](int64_t u, unsigned count) {
+        const dim3 grid(count);
         if(std::min(a.n, a.nb) <= 256)
             hipLaunchKernelGGL((trtri_panel_kernel<T, 4>), grid, dim3(panel::PNT), 0, h->stream, a,
                                panels, u, pw);
         else
             hipLaunchKernelGGL((trtri_panel_kernel<T, 8>), grid, dim3(panel::PNT), 0, h->stream, a,
                                panels, u, pw);
-    }
+    });
     if(!a.A.arr || !a.X.arr)
         return launch_status();
     const int     strips = (std::min(a.n, a.nb) + TS - 1) / TS;
     const int64_t turns  = int64_t(a.batch) * nblk * strips;
-    for(int64_t u = 0; u < turns; u += 1 << 30)
-        hipLaunchKernelGGL(trtri_turn_kernel<T>, dim3(unsigned(std::min<int64_t>(turns - u, 1 << 30))),
-                           dim3(256), 0, h->stream, a, strips, u);
+    for_launch_slices(turns, 256, [&](int64_t u, unsigned count) {
+        hipLaunchKernelGGL(trtri_turn_kernel<T>, dim3(count), dim3(256), 0, h->stream, a, strips, u);
+    });
     return launch_status();
 }
 
