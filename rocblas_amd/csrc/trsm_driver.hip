@@ -317,7 +317,7 @@ size_t trsm_workspace_bytes(const TrsmProblem<T>&)
 template <typename T>
 rocblas_status trsm_launch(rocblas_handle h, const TrsmProblem<T>& p)
 {
-    // a chained launch of an earlier call gave up a wait: report it here
+    // a wait that a kernel of an earlier call gave up: report it here
     if(rocblas_status st = take_async_error(h); st != rocblas_status_success)
         return st;
     DeviceGuard dg(h->device);

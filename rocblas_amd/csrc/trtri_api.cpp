@@ -279,7 +279,7 @@ rocblas_status trtri_core(rocblas_handle    handle,
                           void*             split_ws,
                           size_t            split_bytes)
 {
-    // a split product of an earlier call gave up a wait: report it here
+    // a wait that a kernel of an earlier call gave up: report it here
     if(rocblas_status st = take_async_error(handle); st != rocblas_status_success)
         return st;
     BatchPtr<const T> Asrc = A;

@@ -226,10 +226,13 @@ constexpr int kVbWideInstancesPerCu = 8;
 template <typename T>
 rocblas_status vbatched_launch(rocblas_handle h, VbArgs<T> a)
 {
+    // a wait that a kernel of an earlier call gave up: report it here
+    if(rocblas_status st = take_async_error(h); st != rocblas_status_success)
+        return st;
     DeviceGuard g(h->device);
     a.unit = a.batch / kVbWideInstancesPerCu >= h->num_cus ? 2 * panel::PNC : panel::PNC;
     hipLaunchKernelGGL(vb_plan_kernel<T>, dim3(1), dim3(1024), 0, h->stream, a);
-    rocblas_status st = launch_status();
+    const rocblas_status st = launch_status();
     if(st != rocblas_status_success)
         return st;
     int gmax = 1;

@@ -310,3 +310,39 @@ def test_graph_capture_with_new_sizes(h):
             assert np.abs(got - ref).max() <= 1e-12 * np.abs(ref).max(), (rep, i, m, n)
         _ = (P.dB[0] * 2).sum().item()
     hg.close()
+
+
+def test_wait_timeout_is_reported_by_the_next_call():
+    """A variable-size batch whose waits give up (forced from the host: a few polls and an
+    unreachable target, so every kernel still runs to its end) leaves wrong results: the next call
+    reports it, once, and does no work; the call after that is right."""
+    rng = np.random.default_rng(77)
+    ms, ns = [40, 200, 300, 64], [3, 20, 17, 33]
+    As = [oracle.diag_dominant_triangular(m, "L", rng) for m in ms]
+    Bs = [np.asfortranarray(rng.uniform(-1, 1, (m, n))) for m, n in zip(ms, ns)]
+
+    def problem():
+        return VbProblem("L", ms, ns, [np.nan_to_num(A) for A in As], Bs)
+
+    ht = GpuHandle()
+    try:
+        good = problem()
+        assert good.run(ht, "L", "L", "N", "N", 1.0) == S.success
+        torch.cuda.synchronize()
+        want = [good.result(i) for i in range(4)]
+        assert ht.set_chain_test_timeout(1) == S.success
+        say("vbatched timeout forced")
+        assert problem().run(ht, "L", "L", "N", "N", 1.0) == S.success
+        torch.cuda.synchronize()
+        assert ht.set_chain_test_timeout(0) == S.success
+        p = problem()
+        assert p.run(ht, "L", "L", "N", "N", 1.0) == S.internal_error
+        torch.cuda.synchronize()
+        assert all(np.array_equal(p.result(i), Bs[i]) for i in range(4))
+        say("vbatched after timeout")
+        assert p.run(ht, "L", "L", "N", "N", 1.0) == S.success
+        torch.cuda.synchronize()
+        assert all(np.array_equal(p.result(i), want[i]) for i in range(4))
+        assert ht.get_async_status() == S.success
+    finally:
+        ht.close()
