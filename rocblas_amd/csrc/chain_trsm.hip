@@ -49,9 +49,9 @@ __device__ __forceinline__ void chain_unit(const SmallArgs<T>& a, unsigned* flag
     const T scale = (a.flags & SF_SCALE) ? alpha : T(1);
     if(alpha == T(0))
     {
-        // B := 0 (nobody waits: alpha is uniform); every workgroup a share
-        if(S == 0)
-            panel_zero<T>(Bp, a.K, a.nvec, a.ldb, a.flags, v0, PNC);
+        // B := 0 (nobody waits: alpha is uniform); every workgroup its rows
+        const int r0 = S * 64 * NT;
+        panel_zero<T>(Bp, r0, min(r0 + 64 * NT, a.K), a.nvec, a.ldb, a.flags, v0, PNC);
         return;
     }
     unsigned* const link = flags + p * CHAIN_WORDS;

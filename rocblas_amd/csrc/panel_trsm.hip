@@ -25,7 +25,7 @@ __device__ __forceinline__ void panel_unit(const SmallArgs<T>& a, panel::PanelWa
     const int      v0   = int(unit - b * a.chunks) * panel::PNC * NVG;
     T*             Bp   = a.B.get(b);
     if(alpha == T(0))
-        panel::panel_zero<T>(Bp, a.K, a.nvec, a.ldb, a.flags, v0, panel::PNC * NVG);
+        panel::panel_zero<T>(Bp, 0, a.K, a.nvec, a.ldb, a.flags, v0, panel::PNC * NVG);
     else
     {
         panel::panel_solve<T, NT, NVG, panel::PM_SINGLE>(

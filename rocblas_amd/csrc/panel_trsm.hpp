@@ -255,17 +255,26 @@ __device__ __forceinline__ void store4(T* p, const T (&x)[4])
     *(__attribute__((address_space(1))) v4*)(p) = v4{x[0], x[1], x[2], x[3]};
 }
 
-// B := 0 for nv vectors from v0 (alpha == 0; A is not referenced)
+// Rows i0..i1 - 1 of nv (16 or 32) vectors of B from v0 := 0 (alpha == 0; A is
+// not referenced)
 template <typename T>
-__device__ void panel_zero(T* Bp, int K, int nvec, int ldb, int flags, int v0, int nv)
+__device__ void panel_zero(T* Bp, int i0, int i1, int nvec, int ldb, int flags, int v0, int nv)
 {
-    const bool cols = flags & SF_COLS;
-    for(int e = threadIdx.x; e < K * nv; e += PNT)
+    const int vend = min(v0 + nv, nvec);
+    int       tid  = threadIdx.x;
+    asm volatile("" : "+v"(tid)); // (nothing of this is kept in registers beside a solve)
+    if(flags & SF_COLS)
     {
-        const int i = cols ? e % K : e / nv, v = v0 + (cols ? e / K : e % nv);
-        if(v < nvec)
-            gstore(Bp + (cols ? int64_t(i) + int64_t(v) * ldb : int64_t(v) + int64_t(i) * ldb),
-                   T(0));
+        for(int v = v0 + tid / WAVE; v < vend; v += PNT / WAVE)
+            for(int i = i0 + tid % WAVE; i < i1; i += WAVE)
+                gstore(Bp + (int64_t(i) + int64_t(v) * ldb), T(0));
+    }
+    else
+    {
+        const int lg = nv > PNC ? 5 : 4;
+        const int v  = v0 + (tid & (nv - 1));
+        for(int i = i0 + (tid >> lg); v < vend && i < i1; i += PNT >> lg)
+            gstore(Bp + (int64_t(v) + int64_t(i) * ldb), T(0));
     }
 }
 

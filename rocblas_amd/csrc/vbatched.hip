@@ -202,7 +202,7 @@ __global__ void __launch_bounds__(panel::PNT) __attribute__((amdgpu_waves_per_eu
         {
             const int v0 = p * a.unit;
             if(alpha == T(0))
-                panel::panel_zero<T>(Bp, k, nv, ldb, flags, v0, a.unit);
+                panel::panel_zero<T>(Bp, 0, k, nv, ldb, flags, v0, a.unit);
             else if(a.unit > panel::PNC && nv - v0 > panel::PNC)
                 panel::panel_solve<T, 4, 2, panel::PM_MULTI>(Ap, Bp, k, nv, lda, ldb, flags, alpha,
                                                              v0, vb_smem, pw);
