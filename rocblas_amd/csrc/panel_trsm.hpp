@@ -575,11 +575,16 @@ struct PanelSolver
     // there too.
     __device__ __forceinline__ void solve_unscaled(T (&c)[NVG][4], int t)
     {
-        const int below = PNC * t + g < K ? g : 0;
-        const T*  p     = Ab + int64_t(min(PNC * t + g, K - 1)) * rs + int64_t(PNC * t) * cs;
-        for(int j = 0; j < PNC - 1 && PNC * t + j < K; ++j)
+        // (opaque: what this seldom taken path computes is not to be kept in
+        // registers outside it)
+        int rs_ = rs, cs_ = cs, K_ = K, t_ = t;
+        asm volatile("" : "+s"(rs_), "+s"(cs_), "+s"(K_), "+s"(t_));
+        const int below = PNC * t_ + g < K_ ? g : 0;
+        const T*  p     = Ab + int64_t(min(PNC * t_ + g, K_ - 1)) * rs_ + int64_t(PNC * t_) * cs_;
+        for(int j = 0; j < PNC - 1 && PNC * t_ + j < K_; ++j)
         {
-            const T x = gload(p + int64_t(j) * cs);
+            const T x = gload(p);
+            p += cs_;
 #pragma unroll
             for(int v = 0; v < NVG; ++v)
 #pragma unroll
@@ -651,8 +656,8 @@ struct PanelSolver
         if(__builtin_expect(again != 0, 0))
         {
             T d[NVG][4];
-            // (the right-hand sides are not kept during the steps; opaque
-            // strides, or their wider forms would be kept for the stores too)
+            // (the right-hand sides are not kept during the steps; opaque as in
+            // solve_unscaled)
             int br_ = br, bv_ = bv;
             asm volatile("" : "+s"(br_), "+s"(bv_));
             load_rhs(t, br_, bv_);
