@@ -282,6 +282,7 @@ struct GemmArgsT
     // instance, zero between launches), the error word a given-up wait
     // raises, and the wait controls.
     int                split_ok;
+    int                cold; // the launch before has just written operands (gemm_rule.hpp)
     int                kc;
     // balanced triangular products (gemm_dma_balanced_kernel): the workspace
     // of 2 * split_w partial tiles of 128 x 128 (nullptr: not available), its

@@ -13,6 +13,7 @@
 // diagonal block; such products with few tiles split their tiles' K ranges or
 // balance their K steps over the workgroups.
 #include "device_common.hpp"
+#include "gemm_rule.hpp"
 #include "gemm_tile.hpp"
 
 #include <cstdlib>
@@ -1422,18 +1423,26 @@ static rocblas_status launch_gemm_sel(rocblas_handle h, const GemmArgsT<TA, TB, 
             return launch_gemm_dma_split(h, a);
     }
     // Dense products with few 128 x 128 tiles run on smaller ones
-    // (gemm_tile.hip), which fill the last wave of workgroups better: below
-    // four per CU with 16-byte loads, below two with the 4-byte loads of
-    // unaligned operands, whose issue rate a 128 x 128 tile halves.  Measured
-    // on MI355X, TF/s of 128 x 128 / 64 x 64 tiles: FP64 256 x 16384 x 256 (256
-    // tiles) 37.8 / 49.8, 2048^3 (256) 56.9 / 66.4, 512 x 16384 x 512 (512)
-    // 55.6 / 61.3, unaligned 2048 x 4096 x 2048 (512) 66.7 / 51.3; FP32
-    // unaligned 1465 x 2999 x 1536 (288) 62 / 80.
-    int64_t few = cus;
+    // (gemm_tile.hip) where these pay, which fill the last wave of workgroups
+    // better: below four per CU with 16-byte loads; with 4-byte loads, whose
+    // issue rate a 128 x 128 tile halves, below two (gemm_rule.hpp).  Measured
+    // on MI355X, us of 128 x 128 / 64 x 64 tiles: FP64 2048^3 (256 tiles) 301 /
+    // 251, 3072^3 (576) 1180 / 813, 5120 x 3072 x 1024 (960) 545 / 470; FP32 2048^3
+    // 154 / 139, 2048 x 3072 x 2048 (384) 277 / 204, 3072^3 611 / 441, 4096 x 2048
+    // x 4096 (512) 538 / 519, 5120 x 3072 x 1024 295 / 261; 4-byte loads: FP64 2048
+    // x 3072 x 2048 577 / 502, FP32 340 / 274.
+    int64_t few  = cus;
+    bool    tile = false;
     if constexpr(std::is_same_v<TA, TB> && std::is_same_v<TA, TC>)
     {
-        if(gemm_dma_mode() && gemm_tile_eligible(a))
-            few = gemm_tile_vec16(a) ? 4 * cus : 2 * cus;
+        const bool vec = gemm_tile_vec16(a);
+        tile           = gemm_dma_mode() && gemm_tile_eligible(a)
+               && gemm_tile_pays(sizeof(TA), vec, a.cold, a.opA == 1, a.opB == 1, tiles(64, 64),
+                                 a.K, cus);
+        const bool dma = !vec && gemm_dma_eligible(a, sizeof(TA) == 8 ? 8 : 16)
+                         && gemm_dma_beats_4byte(tiles(128, 128), cus);
+        if(tile)
+            few = vec ? 4 * cus : dma ? cus : 2 * cus;
     }
     if(tiles(128, 128) >= few)
     {
@@ -1482,7 +1491,7 @@ static rocblas_status launch_gemm_sel(rocblas_handle h, const GemmArgsT<TA, TB, 
     }
     if constexpr(std::is_same_v<TA, TB> && std::is_same_v<TA, TC>)
     {
-        if(gemm_dma_mode() && gemm_tile_eligible(a))
+        if(tile)
             return launch_gemm_tile(h, a, tiles(64, 64) >= cus ? 64 : 32);
     }
     if(tiles(64, 64) >= cus)

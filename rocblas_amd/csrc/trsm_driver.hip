@@ -224,6 +224,7 @@ struct Solver
         g.alpha        = T(-1);
         g.beta         = T(1);
         g.skip_if_zero = p.alpha_dev;
+        g.cold         = 1; // B's rows are the solve's of the launch before
         g.batch        = p.batch;
         // block of A holding M[R2, R1] (tA: A[R1, R2]^T)
         const int64_t a_off = tA ? int64_t(R1) + int64_t(R2) * p.lda

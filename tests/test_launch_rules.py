@@ -1,5 +1,6 @@
 """Host-side launch rules, compiled by themselves: launches of more workgroups than one launch can
-have (CPU), and solves and inverses that need them (GPU)."""
+have, which products run on the LDS-load tiles (CPU); solves and inverses that need several launches
+(GPU)."""
 import os
 import shutil
 import subprocess
@@ -38,6 +39,34 @@ def test_slices_cover_every_workgroup_below_the_thread_limit(tmp_path, threads):
             assert int(first) == at and 0 < int(count) * threads < 2**32
             at += int(count)
         assert at == n
+
+
+# (bytes per element, 16-byte loads, in a solve, A and B transposed, 64 x 64 tiles, K) of a product,
+# and its measured time on the LDS-load tiles over the register-staged kernels' (256 CUs), where the
+# two differ by 4% or more
+MEASURED = [
+    (4, 1, 0, 0, 0, 16, 256, 0.79), (4, 1, 0, 0, 0, 64, 64, 0.92), (4, 1, 1, 0, 0, 64, 256, 0.79),
+    (4, 1, 0, 1, 0, 132, 320, 0.72), (4, 1, 0, 0, 0, 256, 1024, 0.49),
+    (4, 0, 0, 0, 0, 63, 48, 1.55), (4, 0, 0, 0, 1, 16, 256, 1.41), (4, 0, 0, 0, 0, 64, 512, 1.44),
+    (4, 0, 0, 0, 1, 64, 1024, 1.28), (4, 0, 0, 1, 0, 100, 320, 1.21), (4, 0, 0, 0, 1, 64, 4096, 0.82),
+    (4, 0, 0, 0, 0, 128, 320, 1.40), (4, 0, 0, 1, 0, 128, 1024, 0.90), (4, 0, 0, 0, 0, 182, 64, 1.14),
+    (4, 0, 0, 1, 0, 182, 1024, 0.83), (4, 0, 0, 0, 0, 256, 64, 0.93), (4, 0, 0, 1, 1, 1024, 256, 0.76),
+    (4, 0, 1, 0, 0, 64, 320, 1.16), (4, 0, 1, 0, 0, 240, 384, 0.86), (4, 0, 1, 0, 0, 64, 1024, 0.92),
+    (8, 1, 0, 0, 0, 16, 64, 0.86), (8, 1, 0, 0, 0, 64, 1024, 0.64), (8, 1, 0, 1, 0, 132, 64, 0.96),
+    (8, 0, 0, 0, 0, 63, 48, 1.34), (8, 0, 0, 1, 0, 16, 256, 1.61), (8, 0, 1, 0, 0, 64, 320, 1.15),
+    (8, 0, 0, 0, 1, 182, 4096, 1.14), (8, 0, 0, 0, 0, 165, 800, 1.12),
+    (8, 0, 0, 0, 0, 256, 1024, 0.94), (8, 0, 0, 1, 0, 256, 1024, 1.05), (8, 0, 0, 0, 0, 506, 64, 0.94),
+    (8, 0, 0, 1, 0, 1024, 256, 0.87)]
+
+
+@pytest.mark.skipif(CXX is None, reason="g++ not available")
+def test_products_run_on_the_kernel_that_measured_faster(tmp_path):
+    body = "".join(f'std::printf("%d\\n", gemm_tile_pays({s}, {v}, {c}, {ta}, {tb}, {t}, {k}, 256));\n'
+                   for s, v, c, ta, tb, t, k, _ in MEASURED)
+    out = run_cpp(tmp_path, body, ["gemm_rule.hpp"])
+    assert len(out) == len(MEASURED)
+    for case, got in zip(MEASURED, out):
+        assert int(got) == (case[-1] < 1), case
 
 
 @pytest.mark.gpu
