@@ -809,6 +809,11 @@ struct PanelSolver
                 early<0>(yf, mine);
             }
         }
+        // (no load of the loops above is in flight from here on: else the
+        // compiler waits for it, and with it for the operands loaded later,
+        // wherever one of its registers is used again)
+        if(MODE == PM_CHAIN || MODE == PM_MULTI)
+            __builtin_amdgcn_s_waitcnt(0x0F70); // vmcnt(0)
         segments<0>(mine);
     }
 
