@@ -604,23 +604,33 @@ struct PanelSolver
         return MODE == PM_INVERSE && t == 0 && j < group_vec(q, r);
     }
 
-    // y_t from the eliminated right-hand sides, and into its LDS slot (negated)
-    __device__ __forceinline__ void scale_y(T (&c)[NVG][4], int t) const
+    // c by dg or -dg: y_t from the eliminated right-hand sides.  Two products
+    // rather than a product and a negation, which takes two instructions in
+    // FP64; only the negated one, for the LDS slot, is on the chain.
+    __device__ __forceinline__ void scale_y(T (&y)[NVG][4], const T (&c)[NVG][4], T by, int t) const
     {
 #pragma unroll
         for(int v = 0; v < NVG; ++v)
 #pragma unroll
             for(int r = 0; r < NR; ++r)
-                c[v][r] = above_unit(t, g, r) ? T(0) : c[v][r] * dg;
+                y[v][r] = c[v][r] * by;
+        if constexpr(MODE == PM_INVERSE)
+            if(t == 0)
+            {
+#pragma unroll
+                for(int r = 0; r < NR; ++r)
+                    y[0][r] = above_unit(t, g, r) ? T(0) : y[0][r];
+            }
     }
-    __device__ __forceinline__ void write_y(const T (&c)[NVG][4], int t) const
+    // -y_t into its LDS slot
+    __device__ __forceinline__ void write_y(const T (&y)[NVG][4], int t) const
     {
         T* p = Y + (t % PRING) * YS + (g ^ kx);
 #pragma unroll
         for(int v = 0; v < NVG; ++v)
 #pragma unroll
             for(int r = 0; r < NR; ++r)
-                p[v * YV + mfma_row<T>(q, r) * YP] = -c[v][r];
+                p[v * YV + mfma_row<T>(q, r) * YP] = y[v][r];
     }
 
     // own sub-block t (tile I) is final: solve, publish, store
@@ -641,16 +651,20 @@ struct PanelSolver
             SolveSteps<T, NVG, NR, 0>::run(c, Ld);
         // A value that is not finite when its step reads it leaves none of its
         // vector finite.  The checks run beside the LDS writes, where they cost
-        // up to 1% of a solve (512 x 256 35.4 -> 35.5 us; in front of the writes
-        // 36.5).
-        scale_y(c, t);
-        write_y(c, t);
+        // the chain nothing (512 x 256 35.4 -> 35.5 us; in front of the writes
+        // 36.5), and up to 5% where many short solves fill the vector units (FP64
+        // 2000 instances 65 x 130 125 -> 130 us).
+        T y[NVG][4];
+        T ndg = -dg;
+        asm volatile("" : "+v"(ndg)); // (not folded into negations)
+        scale_y(y, c, ndg, t);
+        write_y(y, t);
         uint64_t again = scaled ? 0 : 1;
 #pragma unroll
         for(int v = 0; v < NVG; ++v)
 #pragma unroll
             for(int r = 0; r < NR; ++r)
-                again |= __builtin_amdgcn_ballot_w64(not_finite(c[v][r]));
+                again |= __builtin_amdgcn_ballot_w64(not_finite(y[v][r]));
         // the slot is written before the counter says so
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
         if(__builtin_expect(again != 0, 0))
@@ -667,17 +681,18 @@ struct PanelSolver
                 for(int r = 0; r < NR; ++r)
                     d[v][r] = fma(scale, bq[v][r], C[I][v][r]);
             solve_unscaled(d, t);
-            scale_y(d, t);
             // finite results keep their bits whatever their neighbours hold
 #pragma unroll
             for(int v = 0; v < NVG; ++v)
 #pragma unroll
                 for(int r = 0; r < NR; ++r)
-                    c[v][r] = scaled && !not_finite(c[v][r]) ? c[v][r] : d[v][r];
-            write_y(c, t);
+                    c[v][r] = scaled && !not_finite(y[v][r]) ? c[v][r] : d[v][r];
+            scale_y(y, c, ndg, t);
+            write_y(y, t);
             asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
         }
         __hip_atomic_store(done, t + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        scale_y(c, c, dg, t);
         // (opaque, so the addresses are not kept in registers all along)
         int qs = q;
         asm volatile("" : "+v"(qs));
