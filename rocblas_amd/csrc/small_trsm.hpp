@@ -15,10 +15,15 @@
 // constant for each (UPPER, TA) variant.
 //
 // A wavefront serves four slots (instances) of 16 vectors each, also where an
-// instance has fewer vectors: packing more, narrower slots with the triangles
-// in LDS measured slower at every size (FP64, side L, 20000 instances of
-// order 32 with 8 vectors 102 us against 40, order 8 with one vector 11.8
-// against 5.9; one instance of order 32 with 8 vectors 17.4 against 8.6).
+// instance has fewer vectors.  Packing more, narrower slots with the triangles
+// in LDS measured slower up to 20000 instances (FP64, side L: order 32 with 8
+// vectors 102 us against 40, order 8 with one vector 11.8 against 5.9; one
+// instance of order 32 with 8 vectors 17.4 against 8.6) and from order 12 on
+// (200000 of order 12 with 4 vectors 0.53 of the time).  Only several 100000
+// instances of order 8 or less with one to four vectors take longer this way,
+// by up to 11% (FP64, order 4, 3 vectors: 28.9 us against 27.9) or 17% (FP32,
+// order 2, 2 vectors: 23.6 against 20.2), others of them less (0.81 at best): not
+// worth a second kernel.  Four wavefronts per workgroup change nothing there.
 // Every global load of a wavefront is issued before the first wait.
 //
 // Pair order: within a KMAX x KMAX triangle, column c and column KMAX-1-c

@@ -11,8 +11,24 @@ import rocblas_amd as rb
 from rocblas_amd import build as rbuild
 
 EPS = {"d": np.finfo(np.float64).eps, "s": np.finfo(np.float32).eps}
+# 128-row super-blocks on 256 CUs: partial last blocks of 1, 16, 88, 0, 60, 1, 104 and 1 rows
 SHAPES = [(513, 1), (528, 4), (600, 5), (640, 8), (700, 9), (769, 33), (1000, 40), (1025, 3),
-          (1408, 130), (2049, 260)]  # the last two: more than 128 workgroups, then 256-row blocks
+          (1408, 130)]
+# 256-row super-blocks: last blocks of 1, 5 16-row sub-blocks and 3 rows, 255 and 256 rows
+LONG = [2049, 2048 + 16 * 5 + 3, 2048 + 255, 2304]
+
+
+def long_shapes():
+    """LONG with just enough vectors that 128-row blocks would be more workgroups than CUs (the
+    rule of launch_chain), and still few enough for the chained solve (chain_fits)."""
+    import torch
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    out = []
+    for k in LONG:
+        panels, rows64 = cus // (-(-k // 128)) + 1, -(-k // 64)
+        assert panels <= rows64 and rows64 * panels <= 8 * cus
+        out.append((k, 16 * panels - 3))
+    return out
 
 
 @pytest.mark.gpu
@@ -24,7 +40,7 @@ def test_chain_edges_against_oracle(case, prec):
     side, uplo, trans = case
     h = GpuHandle()
     rng = np.random.default_rng(31)
-    for i, (k, nv) in enumerate(SHAPES):
+    for i, (k, nv) in enumerate(SHAPES + long_shapes()):
         m, n = (k, nv) if side == "L" else (nv, k)
         diag, alpha = "NU"[i % 2], (1.0, -0.5)[i % 2]
         print("chain", prec, case, diag, k, nv, flush=True)

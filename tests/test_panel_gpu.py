@@ -104,9 +104,48 @@ def test_badly_scaled_triangles(h, prec, big):
         assert oracle.norm1_rel_diff(k, n, X, ref) <= 40 * EPS[prec] * k
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("op", ["trsm", "trtri"])
+def test_wait_timeout_is_reported_and_heals(op):
+    """Waits inside a panel launch that give up (forced from the host: a few polls and an
+    unreachable target, so every kernel still runs to its end): the next call of the handle reports
+    it once and does no work, the one after that is right."""
+    import torch
+    from tests.gpu_util import GpuHandle
+    rng = np.random.default_rng(9)
+    k, nv = 200, 24
+    A = np.nan_to_num(oracle.diag_dominant_triangular(k, "L", rng))
+    dA = torch.from_numpy(A.ravel(order="F").copy()).cuda()
+    B0 = torch.from_numpy(rng.uniform(-1, 1, k * (nv if op == "trsm" else k))).cuda()
+    hd = GpuHandle()
+
+    def call(B):
+        if op == "trsm":
+            st = rb.trsm(hd, "L", "L", "N", "N", k, nv, 1.0, dA.data_ptr(), k, B.data_ptr(), k)
+        else:
+            st = rb.trtri(hd, "L", "N", k, dA.data_ptr(), k, B.data_ptr(), k)
+        torch.cuda.synchronize()
+        return st, B
+
+    S = rb.rocblas_status
+    st, want = call(B0.clone())
+    assert st == S.success
+    assert hd.set_chain_test_timeout(1) == S.success
+    print("panel timeout forced", op, flush=True)
+    assert call(B0.clone())[0] == S.success
+    assert hd.set_chain_test_timeout(0) == S.success
+    st, B = call(B0.clone())
+    assert st == S.internal_error and torch.equal(B, B0)
+    print("panel after timeout", op, flush=True)
+    st, B = call(B0.clone())
+    assert st == S.success and torch.equal(B, want)
+    assert hd.get_async_status() == S.success
+    hd.close()
+
+
 @pytest.mark.skipif(not os.path.exists(rbuild.HIPCC), reason="hipcc not available")
 def test_every_panel_kernel_has_its_wait_states(tmp_path):
-    """All layouts of the panel solve: no DPP hazard, no scratch."""
+    """All kernels of panel_trsm.hip: no DPP hazard, no scratch."""
     from tests.test_dpp_hazards import compile_asm, kernels, scan
     asm = open(compile_asm(os.path.join(rbuild.CSRC, "panel_trsm.hip"), str(tmp_path / "p.s"))).read()
     found = {name: scan(body) for name, body in kernels(asm, r"panel_\w+kernel")}

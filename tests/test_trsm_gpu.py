@@ -388,7 +388,7 @@ def test_graph_capture_multi_launch_chained_device_mode(h, case):
     pointer mode (alpha read on the device, no synchronisation).  Every replay,
     with eager work between replays, equals the eager result bit for bit."""
     rng = np.random.default_rng(811)
-    m, n, uplo, trans = {"chained": (512, 256, "L", "N"), "recursive": (1500, 700, "U", "T"),
+    m, n, uplo, trans = {"chained": (1024, 256, "L", "N"), "recursive": (1500, 700, "U", "T"),
                          "device_alpha": (700, 40, "L", "T")}[case]
     say("graph", case, m, n)
     A = synth.tri_uniform(m, uplo, 5)
@@ -438,11 +438,11 @@ def test_chained_wait_timeout_is_reported_and_heals(h):
     back at zero, so the following calls -- with more vector panels than the
     failed launch used -- give the normal result."""
     rng = np.random.default_rng(812)
-    m, n = 512, 256
+    m, n, more = 1024, 64, 192  # (above 512 rows: shorter solves are one panel launch)
     A = synth.tri_uniform(m, "L", 8)
-    B0 = np.asfortranarray(rng.uniform(-1, 1, (m, n + 512)))
+    B0 = np.asfortranarray(rng.uniform(-1, 1, (m, n + more)))
     _, want = gpu_trsm(h, "L", "L", "N", "N", m, n, 1.0, A, B0[:, :n].copy(order="F"))
-    _, want_wide = gpu_trsm(h, "L", "L", "N", "N", m, n + 512, 1.0, A, B0)
+    _, want_wide = gpu_trsm(h, "L", "L", "N", "N", m, n + more, 1.0, A, B0)
     dA = dev(A)
     ht = GpuHandle()
     try:
@@ -469,10 +469,10 @@ def test_chained_wait_timeout_is_reported_and_heals(h):
         torch.cuda.synchronize()
         assert np.array_equal(host(dC, (m, n)), want)
         dW = dev(B0)
-        assert rb.trsm(ht, "L", "L", "N", "N", m, n + 512, 1.0, dA.data_ptr(), m, dW.data_ptr(),
+        assert rb.trsm(ht, "L", "L", "N", "N", m, n + more, 1.0, dA.data_ptr(), m, dW.data_ptr(),
                        m) == S.success
         torch.cuda.synchronize()
-        assert np.array_equal(host(dW, (m, n + 512)), want_wide)
+        assert np.array_equal(host(dW, (m, n + more)), want_wide)
         assert ht.get_async_status() == S.success
     finally:
         ht.close()
