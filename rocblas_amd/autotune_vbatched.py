@@ -2,7 +2,7 @@
 
 Sweeps ``panel_groups`` per size bucket of k (<= 64, <= 128, <= 256, larger;
 the last bucket is timed on k in [257, --mhi]) -- how many work items an
-instance is split into (each solves a strided share of its 16-vector panels)
+instance is split into (each solves a strided share of its pieces of 16 or 32 vectors)
 -- each bucket timed on a seeded synthetic workload of its own sizes (default:
 4096 instances, n uniform in [1, 64], side left, lower, no transpose; A with
 diagonal U[1, 2] and off-diagonal U[-1, 1] / m, B uniform in [-1, 1]), then
@@ -59,7 +59,7 @@ def write_header(path, groups, note):
 namespace rbamd
 {{
 // work items per instance of the panel kernel (each a strided share of the
-// instance's 16-vector panels), by size bucket of k: <= 64, <= 128, <= 256,
+// instance's pieces of 16 or 32 vectors), by size bucket of k: <= 64, <= 128, <= 256,
 // larger
 constexpr int kVbPanelBuckets                  = 4;
 constexpr int kVbPanelGroups[kVbPanelBuckets] = {{{", ".join(str(g) for g in groups)}}};

@@ -180,6 +180,7 @@ static rocblas_status launch_small(rocblas_handle h, const SmallArgs<T>& args_in
 constexpr int SMALL_K = 64; // granularity of the recursion's splits
 
 // leaves of the recursion for right-hand sides of at least kWidePanels panels
+// (see Solver::solve)
 constexpr int kWideLeafK  = 256;
 constexpr int kWidePanels = 512;
 
@@ -291,9 +292,13 @@ struct Solver
         // A panel leaf streams its whole triangle once per 16 or 32 vectors and
         // leaves the matrix cores idle along its chain; with many panels the
         // work is better spent in GEMM updates, so wide right-hand sides stop at
-        // leaves of kWideLeafK rows.  Measured with leaves of 256 / 512 rows:
-        // 2048^2 276 / 263 us, FP32 3001 x 2999 626 / 536 us, 16384^2 67.5 / 67.8
-        // ms (leaves of 128: 329 us, 787 us, 68.1 ms).
+        // leaves of kWideLeafK rows.  Measured with leaves of 256 / 512 rows (us,
+        // FP64): 1024 rows with 128 panels of vectors 103 / 97, 192 127 / 112, 256
+        // 132 / 114, 384 186 / 167, 512 207 / 184, 768 302 / 320, 1024 357 / 356; 2048
+        // rows with 128 panels 276 / 263, 256 395 / 359, 384 567 / 529, 512 672 / 624,
+        // 768 987 / 1018, 1024 1312 / 1327; 4096 rows with 768 panels 3580 / 3746.
+        // FP32, 2048 rows: 256 panels 268 / 241, 512 423 / 390, 1024 754 / 723.  So
+        // the line could lie near 700 panels in FP64, and higher in FP32.
         const int64_t panels = int64_t((sideL ? p.n : p.m) + 15) / 16 * p.batch;
         if(panel_fits<T>(h, K) && (K <= kWideLeafK || panels < kWidePanels))
             return panel_leaf(a, b);
@@ -329,8 +334,10 @@ rocblas_status trsm_launch(rocblas_handle h, const TrsmProblem<T>& p)
     const bool  lowerM = (!upperA) != tA;
     const int   K      = sideL ? p.m : p.n;
 
-    // The choice depends on k only, so a batched solve and the single solves
-    // of its instances take the same kernels (and bits).  Triangles of 33 to 64
+    // Up to kPanelMaxK rows the choice depends on k only, so a batched solve and
+    // the single solves of its instances take the same kernels (and bits); above,
+    // the chained solve and the recursion's leaves depend on the vectors and the
+    // batch, and last bits may differ.  Triangles of 33 to 64
     // rows take the panel solve: FP64, side L, against one wavefront walking
     // the triangle through LDS, k = 48 with 64 vectors 25 -> 5.0 us alone and
     // 545 -> 355 us for 20000 instances.
