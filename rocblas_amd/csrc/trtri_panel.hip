@@ -7,8 +7,9 @@
 // the rows above, in the block, as zeros.  The blocks of every instance and all
 // their panels are one launch.
 //
-// In place: pointer arrays that differ may hold the same matrices (strided
-// calls, and pointer arrays that are the same array, read a copy of A).  The
+// In place: pointer arrays that differ may hold the same matrices, and strided
+// batches of different base and stride may meet in an instance (strided calls of
+// one base, and pointer arrays that are the same array, read a copy of A).  The
 // panels of such a block read columns that others solve, so they leave A's
 // triangle alone and write their results below the diagonal transposed into
 // the opposite triangle, which nobody reads; a second launch moves them over.
@@ -122,6 +123,19 @@ __global__ void __launch_bounds__(256) trtri_turn_kernel(const TrtriDiagArgs<T> 
 }
 } // namespace
 
+// Whether an instance's A can be its X: pointer arrays are device data; strided
+// batches that differ in base and stride meet in at most one instance.
+template <typename T>
+static bool may_be_in_place(const TrtriDiagArgs<T>& a)
+{
+    if(a.A.arr || a.X.arr)
+        return a.A.arr && a.X.arr;
+    const int64_t bytes = int64_t(reinterpret_cast<intptr_t>(a.X.base + a.X.offset)
+                                  - reinterpret_cast<intptr_t>(a.A.base + a.A.offset));
+    const int64_t step  = (a.A.stride - a.X.stride) * int64_t(sizeof(T));
+    return step ? bytes % step == 0 && bytes / step >= 0 && bytes / step < a.batch : bytes == 0;
+}
+
 template <typename T>
 rocblas_status trtri_panel_launch(rocblas_handle h, const TrtriDiagArgs<T>& a)
 {
@@ -141,7 +155,7 @@ rocblas_status trtri_panel_launch(rocblas_handle h, const TrtriDiagArgs<T>& a)
             hipLaunchKernelGGL((trtri_panel_kernel<T, 8>), grid, dim3(panel::PNT), 0, h->stream, a,
                                panels, u, pw);
     });
-    if(!a.A.arr || !a.X.arr)
+    if(!may_be_in_place(a))
         return launch_status();
     const int     strips = (std::min(a.n, a.nb) + TS - 1) / TS;
     const int64_t turns  = int64_t(a.batch) * nblk * strips;

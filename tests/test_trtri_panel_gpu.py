@@ -111,3 +111,31 @@ def test_two_pointer_arrays_of_the_same_matrices(uplo, prec):
         # clients/include/unit.hpp:631-638: eps * max(10000, n), relative
         assert np.abs(got[0].T - tri).max() / np.abs(tri).max() <= np.finfo(dt).eps * max(10000, n)
     h.close()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("uplo", ["L", "U"])
+def test_strided_batches_that_meet_in_one_instance(uplo):
+    """A at stride 2 S from 0, invA at stride S from S: the second instance's are the same memory."""
+    import torch
+    from tests.gpu_util import GpuHandle
+    h = GpuHandle()
+    rng = np.random.default_rng(23)
+    for n in (40, 300, 600):
+        print("trtri strided, one instance in place", uplo, n, flush=True)
+        S = n * n
+        mats = [np.nan_to_num(oracle.diag_dominant_triangular(n, uplo, rng)) for _ in range(2)]
+        flat = [torch.from_numpy(M.ravel(order="F").copy()).cuda() for M in mats]
+        buf = torch.zeros(3 * S, dtype=torch.float64, device="cuda")
+        buf[:S], buf[2 * S:] = flat[0], flat[1]
+        base = buf.data_ptr()
+        assert rb.trtri_strided_batched(h, uplo, "N", n, base, n, 2 * S, base + 8 * S, n, S, 2) == 0
+        for i in range(2):
+            want = torch.zeros_like(flat[i])
+            src = flat[i].repeat(2)  # as a batch: the same kernels
+            out = want.repeat(2)
+            assert rb.trtri_strided_batched(h, uplo, "N", n, src.data_ptr(), n, S, out.data_ptr(),
+                                            n, S, 2) == 0
+            assert torch.equal(buf[(i + 1) * S:(i + 2) * S], out[:S]), (n, i)
+        assert torch.equal(buf[:S], flat[0])
+    h.close()
